@@ -22,8 +22,8 @@
 //                up, down and the fused gate|up at M = 2048);
 //   GemmTile128  128 x 128, 4 waves, a ring of 4;
 //   GemmTile64   64 x 128, 4 waves, a ring of 6: where 128-row tiles would
-//                leave CUs idle (the N = 1024 K / V projections at M = 2048,
-//                prompts of at most 64 tokens).
+//                leave CUs idle (the N = 1024 K / V projections at M = 2048).
+// Prompts of up to 160 or 256 rows run gemm_stream.hip instead.
 // When the last round of tiles would leave at least half of the CUs idle,
 // the last tile columns run as tiles of half the height in the same launch
 // (GemmTileWideHalf, 128 x 256, for GemmTileWide; GemmTile128x8 for
@@ -87,61 +87,13 @@
 #include <atomic>
 #include <type_traits>
 
-#include "cascade_device.h"
-#include "cascade_internal.h"
+#include "gemm_common.h"
 
 namespace cascade {
-
-enum GemmEpilogue : int {
-  kGemmStore = 0,
-  kGemmResidual = 1,
-  kGemmQkvRope = 2,
-  kGemmSwiglu = 3,
-  kGemmSilu = 4,
-  kGemmMul = 5,
-  kGemmF32 = 6,
-};
 
 constexpr int kTileN = 128;
 constexpr int kTileK = 64;
 constexpr int kGroupM = 4;
-constexpr int kXcds = 8;
-constexpr int kGemmHead = 128;
-constexpr int kGemmHalfHead = 64;
-
-struct GemmArgs {
-  const uint16_t *x;  // [m, k]
-  const uint16_t *w0;  // store/residual/silu/mul/f32: W; qkv: Wq; swiglu: Wgate
-  const uint16_t *w1;  // qkv: Wk; swiglu: Wup
-  const uint16_t *w2;  // qkv: Wv
-  int64_t n0, n1, n2;  // rows of w0 / w1 / w2 (swiglu: n0 = n_half)
-  int64_t m, k;
-  uint16_t *y;  // [m, ldy] (qkv: the q rows, ldy = n0)
-  int64_t ldy;
-  float *yf;    // kGemmF32 output [m, ldy]
-  const uint16_t *aux;  // residual (kGemmResidual) or gate (kGemmMul), [m, ldy]
-  const uint16_t *rope_cos;  // [positions, 64] bf16
-  const uint16_t *rope_sin;
-  int64_t pos0;
-  uint16_t *k_out;  // position 0 of KV head 0 of this layer's K cache
-  uint16_t *v_out;
-  int64_t kv_head_stride;
-  int64_t slot0;
-  // full tiles: a tiles_m x tiles_n grid (tiles of them, per_xcd on each
-  // XCD); half-height tiles: an htiles_m x htiles_n grid right of it
-  int32_t tiles_m, tiles_n, tiles, per_xcd;
-  int32_t htiles_m, htiles_n, htiles, hper_xcd;
-  int32_t vec_out;  // row pitches and widths allow 16-byte output accesses
-  // split K (fp32 partials, kGemmF32 only): workgroup row blockIdx.y runs
-  // slabs [blockIdx.y * split_slabs, + split_slabs) of K and writes its
-  // partial at yf + blockIdx.y * split_stride; 0: the whole K
-  int32_t split_slabs;
-  int64_t split_stride;
-};
-
-__device__ __forceinline__ float gemm_silu(float g) {
-  return g / (1.0f + expf(-g));
-}
 
 // Tile (tm, tn) of logical tile t in a tiles_m x tiles_n grid (false:
 // padding workgroup, no work).  Logical tiles run in groups of kGroupM
@@ -197,12 +149,10 @@ __device__ __forceinline__ int gemm_col(int wn, int j, int lr) {
   return 16 * T::H * wn + 16 * (j % T::H) + 64 * (j / T::H) + lr;
 }
 
-// only_j >= 0: store only fragment column only_j (the element-wise
-// epilogues; RoPE and SwiGLU pair fragment j with j + H and need both).
 template <int EPI, class T>
 __device__ __forceinline__ void gemm_epilogue(
     const GemmArgs &a, int tm, int tn, int wm, int wn, int lane,
-    const f32x4 (&acc)[T::FM][T::FN], int only_j = -1) {
+    const f32x4 (&acc)[T::FM][T::FN]) {
   const int lr = lane & 15;
   const int lq = lane >> 4;
 #pragma unroll
@@ -258,7 +208,6 @@ __device__ __forceinline__ void gemm_epilogue(
       } else {
 #pragma unroll
         for (int j = 0; j < T::FN; ++j) {
-          if (only_j >= 0 && j != only_j) continue;
           const int64_t col =
               static_cast<int64_t>(tn) * kTileN + gemm_col<T>(wn, j, lr);
           if (col >= a.n0) continue;
@@ -765,7 +714,7 @@ __global__ __launch_bounds__(T::WAVES *kWave) void gemm_kernel(GemmArgs a) {
 }
 
 // CUs of the device a stream runs on (cached per device; 256 on MI355X).
-static int gemm_device_cus(hipStream_t s) {
+int gemm_device_cus(hipStream_t s) {
   constexpr int kMaxDevices = 64;
   static std::atomic<int> cached[kMaxDevices];
   int dev = 0;
@@ -823,239 +772,6 @@ static hipError_t launch_tiles(GemmArgs &a, int64_t tiles_n, int cus, hipStream_
                        dim3(T::WAVES * kWave), 0, s, a);
 }
 
-// Short prompts (M <= 64 rows, or up to 256 over few columns).  The weights are nearly all the traffic, so
-// they must stream at HBM rate, which needs long runs of one row per load
-// (64-byte pieces of 16 rows per instruction, the layout of an MFMA operand,
-// stream at only 2-3 TB/s).  A workgroup computes one pair of 16-column
-// fragments of a 128-column tile (the columns of wave column wn of a
-// GemmTile<MR, 1, 4>, so the epilogues' pairing of column c with c + 64
-// holds), or for the element-wise epilogues one fragment of it where the
-// pairs would leave CUs idle (NF = 1: M = 16, o_proj 17.2 -> 12.2 us,
-// down_proj 36.3 -> 28.5 us), for a block of MR rows (grid.y: the row block; M > 64 runs
-// blocks of 64 rows side by side, each reading the column pair's W
-// again, from the XCD's L2 when the blocks share an XCD).  K is walked in slabs through a ring of LDS
-// buffers: every load instruction moves 1 KiB, one or two whole row runs
-// of a slab (the 32 W rows and the MR X rows; rows past M or past a matrix
-// read as zeros through the buffer bounds, and K past a short last slab
-// is never used), each instruction's kilobyte lands after 16 bytes of
-// padding so the fragment reads of 16 rows spread over the banks, and each
-// wave runs the MFMAs of its quarter of a slab's K.  The waves' fp32 partials are summed through LDS in wave
-// order and wave 0 runs the element-wise epilogue.
-template <int MR, int NF = 2>
-struct SkinnyShape {
-  using T = GemmTile<MR, 1, 4>;  // one 16 x 32 column pair of MR rows per workgroup
-  static_assert(NF == 1 || NF == 2, "a column pair or one fragment of it");
-  static constexpr int SLAB_K = MR == 16 ? 512 : 256;
-  static constexpr int RUN = SLAB_K * 2;          // bytes of one row in a slab
-  static constexpr int RPI = 1024 / RUN;          // rows per load instruction (1 KiB)
-  static constexpr int LINE = 1024 + 16;          // LDS pitch of one instruction's rows
-  static constexpr int WROWS = 16 * NF;           // W rows of the fragment(s)
-  static constexpr int SLAB_ROWS = WROWS + MR;    // W rows, then X rows
-  static constexpr int STAGES = 3;
-  static constexpr int WAVES = 4;
-  static constexpr int LOADS = SLAB_ROWS / RPI / WAVES;  // per wave and slab
-  static_assert(SLAB_ROWS % (RPI * WAVES) == 0, "whole instructions per wave");
-  static_assert(16 % RPI == 0, "an instruction's rows stay in one operand");
-};
-// Prompt rows the skinny kernels cover.  A 128-row shape (128-deep slabs,
-// 256-byte runs) measured slower than 64-row tiles at M = 128 (the layer
-// of seven projections 0.460 against 0.311 ms).
-constexpr int kSkinnyRows = 64;
-
-// Slab row r (W rows of fragments 0 and 1, then X rows) sits at LDS byte
-// (r / RPI) * LINE + (r % RPI) * RUN of its buffer.  With 512-byte runs two
-// rows share one 1 KiB line, so a fragment read (16 rows) meets each bank
-// group twice; with 1 KiB runs, once.
-template <int EPI, int MR, int NF = 2>
-__global__ __launch_bounds__(SkinnyShape<MR>::WAVES *kWave) void gemm_skinny_kernel(GemmArgs a) {
-  using S = SkinnyShape<MR, NF>;
-  using T = typename S::T;
-  static_assert(S::WAVES == SkinnyShape<MR>::WAVES, "one workgroup size");
-  static_assert(NF == 2 || (EPI != kGemmQkvRope && EPI != kGemmSwiglu),
-                "RoPE and SwiGLU pair fragment j with j + 1");
-  constexpr int kSlabBytes = S::SLAB_ROWS / S::RPI * S::LINE;
-  __shared__ __attribute__((aligned(16))) unsigned char ring[S::STAGES * kSlabBytes];
-  static_assert(S::WAVES * T::FM * NF * kWave * sizeof(f32x4) <= sizeof(ring),
-                "the reduction fits in the ring");
-  // NF = 2: workgroup x holds the fragment pair of wave column x % 4 of
-  // tile x / 4; NF = 1: fragment (x / 4) % 2 of wave column x % 4 of tile
-  // x / 8 (twice the workgroups for the same columns)
-  constexpr int kPerTile = T::WN * (2 / NF);
-  const int tn = static_cast<int>(blockIdx.x) / kPerTile;
-  const int wn = static_cast<int>(blockIdx.x) % T::WN;
-  const int jsel = NF == 2 ? 0 : (static_cast<int>(blockIdx.x) % kPerTile) / T::WN;
-  const int rb = static_cast<int>(blockIdx.y);  // block of MR rows of X
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int lr = lane & 15;
-  const int g4 = lane >> 4;
-  const int64_t row_bytes = a.k * 2;
-
-  // the matrix, and the row in it, of W slab row r (r < 32: fragment r / 16,
-  // tile column gemm_col(wn, r / 16, r % 16)); rows past a matrix read as
-  // zeros through its buffer bounds
-  auto w_row = [&](int r, const uint16_t *&base, int64_t &rows) -> int64_t {
-    const int j = NF == 2 ? r / 16 : jsel;
-    const int tc = gemm_col<T>(wn, j, r % 16);
-    if constexpr (EPI == kGemmSwiglu) {
-      base = tc < kGemmHalfHead ? a.w0 : a.w1;
-      rows = a.n0;
-      return static_cast<int64_t>(tn) * kGemmHalfHead + (tc % kGemmHalfHead);
-    } else if constexpr (EPI == kGemmQkvRope) {
-      const int64_t hq = a.n0 / kGemmHead, hk = a.n1 / kGemmHead;
-      if (tn < hq) {
-        base = a.w0; rows = a.n0; return static_cast<int64_t>(tn) * kGemmHead + tc;
-      }
-      if (tn < hq + hk) {
-        base = a.w1; rows = a.n1; return (tn - hq) * kGemmHead + tc;
-      }
-      base = a.w2; rows = a.n2; return (tn - hq - hk) * kGemmHead + tc;
-    } else {
-      base = a.w0; rows = a.n0; return static_cast<int64_t>(tn) * kTileN + tc;
-    }
-  };
-  // this wave's load instructions: a buffer over the operand's matrix and
-  // the lane's byte offset of slab 0 (its row of the instruction, then
-  // 16 bytes a lane along that row)
-  constexpr int kLanesPerRow = kWave / S::RPI;
-  u32x4 rsrc[S::LOADS];
-  int voff[S::LOADS];
-#pragma unroll
-  for (int t = 0; t < S::LOADS; ++t) {
-    const int r0 = (wave * S::LOADS + t) * S::RPI;
-    const uint16_t *base;
-    int64_t rows, row;
-    if (r0 < S::WROWS) {
-      row = w_row(r0, base, rows);
-    } else {
-      base = a.x; rows = a.m; row = static_cast<int64_t>(rb) * MR + r0 - S::WROWS;
-    }
-    rsrc[t] = buffer_rsrc_words(base, rows * row_bytes);
-    voff[t] = static_cast<int>((row + lane / kLanesPerRow) * row_bytes) +
-              16 * (lane % kLanesPerRow);
-  }
-  const uint32_t ring_lds = lds_address(ring);
-  const int slabs = static_cast<int>((a.k + S::SLAB_K - 1) / S::SLAB_K);
-  auto load_slab = [&](int slab, int buf) {
-    const uint32_t dst = ring_lds + static_cast<uint32_t>(buf * kSlabBytes);
-#pragma unroll
-    for (int t = 0; t < S::LOADS; ++t)
-      dma_lds16(rsrc[t], voff[t] + slab * S::RUN, dst + (wave * S::LOADS + t) * S::LINE);
-  };
-
-  // fragment reads: lane (lr, g4) of 32-deep chunk q reads row lr of the
-  // operand's 16-row group, bytes 64 q + 16 g4 of its run
-  auto row_at = [&](int r) { return (r / S::RPI) * S::LINE + (r % S::RPI) * S::RUN; };
-  f32x4 acc[T::FM][NF];
-#pragma unroll
-  for (int i = 0; i < T::FM; ++i)
-#pragma unroll
-    for (int j = 0; j < NF; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  constexpr int kChunks = S::SLAB_K / 32 / S::WAVES;  // per wave and slab
-  auto compute = [&](int slab, int buf) {
-    const unsigned char *b0 = ring + buf * kSlabBytes + 16 * g4;
-    const int valid = static_cast<int>(
-        min<int64_t>(S::SLAB_K, a.k - static_cast<int64_t>(slab) * S::SLAB_K) / 32);
-#pragma unroll
-    for (int q = 0; q < kChunks; ++q) {
-      const int chunk = wave * kChunks + q;
-      if (chunk >= valid) break;  // wave-uniform: the last slab of a short K
-      u32x4 xa[T::FM], wb[NF];
-#pragma unroll
-      for (int i = 0; i < T::FM; ++i)
-        xa[i] = *reinterpret_cast<const u32x4 *>(b0 + row_at(S::WROWS + 16 * i + lr) +
-                                                 64 * chunk);
-#pragma unroll
-      for (int j = 0; j < NF; ++j)
-        wb[j] = *reinterpret_cast<const u32x4 *>(b0 + row_at(16 * j + lr) + 64 * chunk);
-#pragma unroll
-      for (int i = 0; i < T::FM; ++i)
-#pragma unroll
-        for (int j = 0; j < NF; ++j) acc[i][j] = mfma_16x16x32_bf16(xa[i], wb[j], acc[i][j]);
-    }
-  };
-  // slab s in buffer s % STAGES; step s waits for this wave's loads of
-  // slab s (the later slabs' loads may stay in flight), one barrier
-  // publishes it and frees slab s - 1's buffer, which takes slab
-  // s + STAGES - 1 (past the end: the last slab again, never read)
-  constexpr int kWaitStep = waitcnt_imm((S::STAGES - 2) * S::LOADS, 0);
-#pragma unroll
-  for (int p = 0; p < S::STAGES - 1; ++p) load_slab(min(p, slabs - 1), p);
-  int buf = 0;
-  for (int slab = 0; slab < slabs; ++slab) {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(kWaitStep);
-    __builtin_amdgcn_s_barrier();
-    const int refill = buf == 0 ? S::STAGES - 1 : buf - 1;
-    load_slab(min(slab + S::STAGES - 1, slabs - 1), refill);
-    compute(slab, buf);
-    buf = buf + 1 == S::STAGES ? 0 : buf + 1;
-  }
-  // every load landed and every LDS read done before the ring holds the
-  // partials
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
-  __syncthreads();
-  f32x4(*partial)[T::FM * NF][kWave] =
-      reinterpret_cast<f32x4(*)[T::FM * NF][kWave]>(ring);
-#pragma unroll
-  for (int i = 0; i < T::FM; ++i)
-#pragma unroll
-    for (int j = 0; j < NF; ++j) partial[wave][i * NF + j][lane] = acc[i][j];
-  __syncthreads();
-  if (wave != 0) return;
-  // the wave partials in wave order, into the pair's fragment slots
-  f32x4 out[T::FM][T::FN];
-#pragma unroll
-  for (int i = 0; i < T::FM; ++i)
-#pragma unroll
-    for (int j = 0; j < T::FN; ++j) out[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int i = 0; i < T::FM; ++i)
-#pragma unroll
-    for (int j = 0; j < NF; ++j) {
-      f32x4 sum = partial[0][i * NF + j][lane];
-      for (int w = 1; w < S::WAVES; ++w) sum += partial[w][i * NF + j][lane];
-      if (NF == 2) {
-        out[i][j] = sum;
-      } else {  // no register array indexed at run time
-        out[i][0] = jsel == 0 ? sum : out[i][0];
-        out[i][1] = jsel == 1 ? sum : out[i][1];
-      }
-    }
-  gemm_epilogue<EPI, T>(a, rb, tn, 0, wn, lane, out, NF == 2 ? -1 : jsel);
-}
-
-template <int EPI>
-static hipError_t launch_skinny(GemmArgs &a, int64_t tiles_n, hipStream_t s) {
-  const int64_t pairs = tiles_n * 4;  // one workgroup per column pair
-  if (pairs > (int64_t{1} << 29)) return static_cast<hipError_t>(CASCADE_ESHAPE);
-  const unsigned blocks = a.m <= 16 ? 1u : static_cast<unsigned>((a.m + 63) / 64);
-  // where the column pairs would leave CUs idle (o_proj / down_proj,
-  // N = 4096: 128 pairs), the element-wise epilogues split each pair over
-  // two workgroups, one fragment each; RoPE and SwiGLU keep their pairs
-  constexpr bool kSplittable = EPI != kGemmQkvRope && EPI != kGemmSwiglu;
-  const bool split = kSplittable && 2 * pairs * blocks <= gemm_device_cus(s);
-  const unsigned grid = static_cast<unsigned>(split ? 2 * pairs : pairs);
-  if constexpr (kSplittable) {
-    if (split) {
-      if (a.m <= 16)
-        return launch_kernel(gemm_skinny_kernel<EPI, 16, 1>, dim3(grid),
-                             dim3(SkinnyShape<16, 1>::WAVES * kWave), 0, s, a);
-      return launch_kernel(gemm_skinny_kernel<EPI, 64, 1>, dim3(grid, blocks),
-                           dim3(SkinnyShape<64, 1>::WAVES * kWave), 0, s, a);
-    }
-  }
-  if (a.m <= 16)
-    return launch_kernel(gemm_skinny_kernel<EPI, 16>, dim3(grid),
-                         dim3(SkinnyShape<16>::WAVES * kWave), 0, s, a);
-  // blocks of 64 rows side by side (grid.y); with an even pair count the
-  // blocks of one column pair run on one XCD (linear index mod 8) and share
-  // its W slabs through that XCD's L2
-  return launch_kernel(gemm_skinny_kernel<EPI, 64>, dim3(grid, blocks),
-                       dim3(SkinnyShape<64>::WAVES * kWave), 0, s, a);
-}
-
 // Schedule of launch_tiles in rounds: whole rounds of full tiles, then a
 // round of half-height tiles (tail 1), a partial round of full tiles
 // (tail 2) or nothing (tail 0).
@@ -1074,27 +790,22 @@ static TileRounds tile_rounds(int64_t tiles_m, int64_t tiles_n, int64_t htiles_m
   return {tiles / cus, 2};
 }
 
-// At most 64 rows of X, or at most 256 over few columns: the skinny
-// kernels.  Else 256-row tiles when there are at least as many as CUs: 256
+// Short prompts: the streaming kernel (gemm_stream.hip).  Else 256-row tiles
+// when there are at least as many as CUs: 256
 // columns wide where their schedule is shorter (below), else 128 wide (a
 // partial last round runs as 128-row half tiles); else 128-row tiles (a
 // partial last round as 64-row half tiles),
 // unless there are fewer of those than CUs and 64-row tiles need no more
 // than twice their rounds: then 64-row tiles (the K / V projections,
-// N = 1024, at M = 2048, and short prompts).
+// N = 1024, at M = 2048).
 template <int EPI>
 static hipError_t launch_gemm(GemmArgs &a, int64_t tiles_n, hipStream_t s) {
-  if (a.m <= kSkinnyRows) return launch_skinny<EPI>(a, tiles_n, s);
   const int cus = gemm_device_cus(s);
-  // up to 256 rows over few columns: blocks of 64 rows through the skinny
-  // kernel while that stays within one workgroup per CU (M = 128: q / o /
-  // down_proj 30 -> 21, 32 -> 22, 103 -> 56 us; k / v up to M = 256 29 ->
-  // 18 us); past that, tiles (M = 192, q_proj: 35 us skinny, 30 tiled).
-  // Not for q|k|v, so that its per-matrix launches (matrix granularity)
-  // sum in the same order as the fused one and match it bit for bit.
-  if (EPI != kGemmQkvRope && a.m <= 4 * kSkinnyRows &&
-      (a.m + kSkinnyRows - 1) / kSkinnyRows * tiles_n * 4 <= cus)
-    return launch_skinny<EPI>(a, tiles_n, s);
+  const int64_t n = EPI == kGemmQkvRope  ? a.n0 + a.n1 + a.n2
+                    : EPI == kGemmSwiglu ? 2 * a.n0
+                                         : a.n0;
+  const StreamPlan sp = stream_plan(EPI, a.m, n, cus);
+  if (sp.fm) return launch_stream(EPI, sp, a, s);
   const int64_t tiles256 = (a.m + 255) / 256 * tiles_n;
   if (a.m > 128 && tiles256 >= cus) {
     // 256 x 256 tiles read a quarter less X and W per MFMA but need 32-deep
@@ -1132,7 +843,7 @@ static hipError_t launch_gemm(GemmArgs &a, int64_t tiles_n, hipStream_t s) {
   // 62.6 -> 45.1 us)
   const int64_t rounds64 = ((a.m + 63) / 64 * tiles_n + cus - 1) / cus;
   const int64_t rounds128 = (tiles128 + cus - 1) / cus;
-  if (a.m <= 64 || (tiles128 < cus && 2 * rounds128 > rounds64))
+  if (tiles128 < cus && 2 * rounds128 > rounds64)
     return launch_tiles<EPI, kTileK, GemmTile64, 6>(a, tiles_n, cus, s);
   return launch_tiles<EPI, kTileK, GemmTile128, 4, GemmTile64, 6>(a, tiles_n, cus, s);
 }
@@ -1163,41 +874,47 @@ static int gemm_check_w(const void *w, int64_t n, int64_t granule, int64_t k) {
 using namespace cascade;
 
 // Split K.  Where 256-row tiles would keep at most half of the CUs busy
-// (prompts of 17 to about 1000 rows over N = 4096: down_proj, and o_proj up
-// to 128 rows; M = 256, down_proj: 102.7 -> 46.1 us, M = 1024: 136.5 ->
-// 110.7 us, o_proj at M = 65: 28.5 -> 19.2 us), K is
-// split over up to kSplitMax rows of workgroups (blockIdx.y), each writing
+// (prompts of 17 to about 1000 rows over N = 4096: down_proj), K is
+// split over up to kSplitMax rows of workgroups, each writing
 // an fp32 partial tile into the caller's workspace; a second launch sums
 // the partials in split order and applies the element-wise epilogue at the
 // same rounding points as the one-pass tile (bf16(sum), then the residual
 // add).  The partials associate the K sum differently from one pass, so a
 // result may differ from the one-pass tile in the last bf16 place, within
-// the same rounding bound.
+// the same rounding bound.  Up to 256 rows the streaming kernel writes the
+// partials (stream_split_plan), past that the 256-row tiles.  Over a short K
+// (K < 8192: o_proj) up to 128 rows the one-pass streaming kernel ends
+// before a split launch and its reduction (M = 64: 13.8 against 15.2 us),
+// so the workspace those shapes ask for is checked and left alone.
 constexpr int kSplitMax = 8;
 constexpr int kSplitMinSlabs = 8;  // 64-deep slabs per split, at least
+constexpr int kShortPrompt = 128;
 
 struct SplitPlan {
   int splits;  // 1: no split
   int per;     // slabs per split
+  StreamPlan stream;  // fm: the streaming kernel writes the partials
 };
 
 static SplitPlan split_plan(int64_t m, int64_t n, int64_t k, int cus) {
-  SplitPlan p{1, 0};
-  // 16 rows and fewer: one skinny block per column pair streams the weight
-  // faster (M = 16, down_proj: 28.6 us one pass, 31.8 split; M = 24: 42.0
-  // against 32.2, M = 64: 51.1 against 34.4)
+  SplitPlan p{1, 0, {0, 0, 1}};
+  // 16 rows and fewer: one pass streams the weight faster (M = 6,
+  // down_proj: 23.3 us one pass, 21 + 4.7 split)
   if (m <= 16 || n % 8 != 0 || k % kTileK != 0) return p;
-  // short K past the skinny blocks: the one-pass 64-row tiles finish first
+  // short K past 128 rows: one pass finishes first
   // (o_proj, M = 192..1024: 22.0..33.8 us one pass, 23.3..42.8 split)
-  if (k < 8192 && m > 2 * kSkinnyRows) return p;
+  if (k < 8192 && m > kShortPrompt) return p;
   const int64_t tiles = (m + 255) / 256 * ((n + kTileN - 1) / kTileN);
   if (2 * tiles > cus) return p;
   const int64_t slabs = k / kTileK;
-  const int64_t sp = std::min<int64_t>(std::min<int64_t>(kSplitMax, cus / tiles),
-                                       slabs / kSplitMinSlabs);
+  int64_t sp = std::min<int64_t>(std::min<int64_t>(kSplitMax, cus / tiles),
+                                 slabs / kSplitMinSlabs);
   if (sp < 2) return p;
+  p.stream = stream_split_plan(m, n, k, cus);
+  if (p.stream.fm) sp = p.stream.splits;
   const int64_t per = (slabs + sp - 1) / sp;
   p.splits = static_cast<int>((slabs + per - 1) / per);  // no empty split
+  p.stream.splits = p.splits;
   p.per = static_cast<int>(per);
   return p;
 }
@@ -1244,8 +961,10 @@ static int gemm_split_k(const GemmArgs &a, const SplitPlan &p, void *ws,
   b.ldy = a.n0;
   b.split_slabs = p.per;
   b.split_stride = part;
-  hipError_t e = launch_tiles<kGemmF32, kTileK, GemmTile256, 3>(
-      b, (a.n0 + kTileN - 1) / kTileN, gemm_device_cus(s), s, p.splits);
+  hipError_t e = p.stream.fm
+                     ? launch_stream(kGemmF32, p.stream, b, s)
+                     : launch_tiles<kGemmF32, kTileK, GemmTile256, 3>(
+                           b, (a.n0 + kTileN - 1) / kTileN, gemm_device_cus(s), s, p.splits);
   if (e != hipSuccess) return e;
   GemmArgs r = a;
   r.yf = static_cast<float *>(ws);
@@ -1327,6 +1046,11 @@ static int gemm_ws(int epi, const void *x, const void *w, const void *aux,
   a.y = static_cast<uint16_t *>(y);
   a.ldy = n;
   a.aux = static_cast<const uint16_t *>(aux);
+  if (k < 8192) {  // m <= kShortPrompt
+    if (workspace_bytes < static_cast<size_t>(p.splits) * m * n * sizeof(float))
+      return CASCADE_EWORKSPACE;
+    return gemm_plain(epi, x, w, aux, y, m, n, k, stream);
+  }
   return epi == kGemmResidual
              ? gemm_split_k<kGemmResidual>(a, p, workspace, workspace_bytes, s)
              : gemm_split_k<kGemmStore>(a, p, workspace, workspace_bytes, s);

@@ -1,0 +1,93 @@
+"""Streaming GEMM of short prompts (gemm_stream.hip) at the edges of its
+shapes: token counts at both sides of each fragment and plan boundary, weight
+rows that do not fill the last workgroup, odd pitches (element-wise stores),
+K below, at and past whole slabs.  Bound of a bf16 product as in
+test_gpu_prefill.py: one bf16 ulp plus 2^-22 sum |x w| of fp32 accumulation.
+"""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from layer_streaming import _hip
+from oracle import cases
+from oracle import llama_oracle as ref
+from test_gpu_prefill import linear_bound_report
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 4096, 64), (15, 16, 128), (16, 4097, 192), (17, 6144, 320),
+    (48, 1024, 1088), (49, 1003, 256), (64, 28672, 64), (65, 4096, 576),
+    (112, 4100, 192), (113, 4096, 448), (159, 8191, 128), (160, 30000, 64),
+    (161, 4096, 320), (256, 6100, 192), (129, 7000, 64)])
+def test_stream_gemm_edges(gpu_device, m, n, k):
+    print("stream gemm m={} n={} k={}".format(m, n, k), flush=True)
+    dev = gpu_device
+    x, w = cases.normal_bf16((m, k), 301), cases.normal_bf16((n, k), 302, 0.05)
+    res = cases.normal_bf16((m, n), 303)
+    xd, wd = x.to(dev), w.to(dev)
+    # rows around the output stay as they were
+    guard = torch.full((m + 2, n), 7.0, dtype=BF16, device=dev)
+    y = torch.empty((m, n), dtype=BF16, device=dev)
+    _hip.gemm(xd, wd, y)
+    assert linear_bound_report(y, x, w) <= 1.0
+    if (n * 2) % 16 == 0:
+        inner = guard[1:m + 1]
+        _hip.gemm_residual(xd, wd, res.to(dev), inner)
+        assert torch.equal(inner, res.to(dev) + y)
+        assert bool((guard[0] == 7.0).all()) and bool((guard[m + 1] == 7.0).all())
+    yf = torch.empty((m, n), dtype=torch.float32, device=dev)
+    _hip.gemm_f32out(xd, wd, yf)
+    if m <= 128:
+        assert torch.equal(yf.to(BF16), y)
+    else:  # logits of more rows run on tiles, whose sums add in another order
+        assert linear_bound_report(yf.to(BF16), x, w) <= 1.0
+
+
+@pytest.mark.parametrize("m,n,k", [(16, 64, 64), (33, 2048, 320), (81, 2112, 576),
+                                   (160, 14336, 256), (97, 14400, 192)])
+def test_stream_swiglu_edges(gpu_device, m, n, k):
+    print("stream swiglu m={} n={} k={}".format(m, n, k), flush=True)
+    dev = gpu_device
+    x = cases.normal_bf16((m, k), 311)
+    wg, wu = (cases.normal_bf16((n, k), s, 0.05) for s in (312, 313))
+    xd, wgd, wud = x.to(dev), wg.to(dev), wu.to(dev)
+    fused, gate, split = (torch.empty((m, n), dtype=BF16, device=dev) for _ in range(3))
+    _hip.gate_up_swiglu_gemm(xd, wgd, wud, fused)
+    _hip.gate_silu_gemm(xd, wgd, gate)
+    _hip.up_mul_gemm(xd, wud, gate, split)
+    assert torch.equal(fused, split)
+    r = cases.compare(fused, F.silu(ref.linear(x, wg)) * ref.linear(x, wu))
+    assert r["ok"], r
+
+
+@pytest.mark.parametrize("m", [1, 17, 49, 160, 161, 256])
+def test_stream_qkv_split_equals_fused(gpu_device, m):
+    # q, k and v as three launches (other weight rows per workgroup) add in
+    # the same order; the last workgroup of the fused launch crosses from k
+    # to v heads when 24 or 48 rows do not divide a matrix
+    dev = gpu_device
+    k, cap = 192, m + 3
+    x = cases.normal_bf16((m, k), 321).to(dev)
+    w = [cases.normal_bf16((rows, k), 322 + i, 0.05).to(dev)
+         for i, rows in enumerate((4096, 1024, 1024))]
+    inv = ref.llama3_inv_freq(128)
+    c, s = ref.rope_cos_sin(inv, list(range(cap)))
+    c, s = c[:, :64].contiguous().to(dev), s[:, :64].contiguous().to(dev)
+    outs = []
+    for groups in ([w], [[w[0], None, None], [None, w[1], None], [None, None, w[2]]]):
+        q = torch.zeros((m, 4096), dtype=BF16, device=dev)
+        kc = torch.zeros((8, cap, 128), dtype=BF16, device=dev)
+        vc = torch.zeros_like(kc)
+        for wq, wk, wv in groups:
+            _hip.qkv_rope_gemm(x, wq, wk, wv, c, s, 2, q, kc.view(-1), vc.view(-1),
+                               cap * 128, 1)
+        outs.append((q, kc, vc))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+    v = ref.linear(x.cpu(), w[2].cpu()).view(m, 8, 128).transpose(0, 1)
+    assert cases.compare(outs[0][2][:, 1:m + 1].cpu(), v)["ok"]
+    assert int(outs[0][2][:, 0].abs().sum()) == 0
