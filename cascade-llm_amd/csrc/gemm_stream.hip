@@ -23,7 +23,9 @@
 // SwiGLU launches (and the logits of a whole vocabulary) start each tile at
 // another run of K: with every CU on the same columns of rows 8 KB apart
 // the same few channels serve all of them (112 rows a CU, loads alone:
-// 44.9 -> 36.2 us).
+// 44.9 -> 36.2 us).  The runs differ between the tiles of one XCD (tile / 8):
+// taken from the tile number itself they agree within an XCD (logits of
+// 26 rows: 259 us, 217 without any, 174 so).
 //
 // Weights are the A operand, tokens the B operand: a lane then holds 4
 // consecutive weight rows, i.e. output columns, of one token.  8-row blocks
@@ -39,7 +41,7 @@
 // gate|up 70.1 -> 39.5 (5.9 TB/s), q|k|v 23.1 -> 15.5, o_proj 16.8 -> 13.0,
 // down_proj (4 runs of K) 31.3 -> 27.6 with the reduction; M = 157 gate|up
 // 73.6 -> 59.2, q|k|v 28.7 -> 22.7, o_proj 27.9 -> 17.1, k / v 18 -> 10.7;
-// M = 26 logits of 128256 rows 259 -> 172.
+// M = 26 logits of 128256 rows 259 -> 168.
 #include <algorithm>
 #include <type_traits>
 
@@ -62,7 +64,11 @@ struct StreamShape {
   static constexpr int NI = ROWS / RPI;       // and all
   static constexpr int PER = (NI + WAVES - 1) / WAVES;
   static constexpr int SLAB = ROWS * RB;
-  static constexpr int FIT = 151552 / SLAB;
+  // the logits of a whole vocabulary take several rounds of workgroups: two
+  // of them share a CU where 3 slabs each fit, one loading while the other
+  // starts or stores (M = 26: 174 -> 168 us, M = 64: 194 -> 187)
+  static constexpr bool TWO = NR == 128 && 2 * 3 * SLAB <= 158000;
+  static constexpr int FIT = (TWO ? 79000 : 151552) / SLAB;
   static constexpr int STAGES = FIT > 12 ? 12 : FIT;
   static constexpr int PITCH = 16 * FN + 4;   // floats per token of the staged tile
   static constexpr int LDS = std::max(STAGES * SLAB, MT * PITCH * 4);
@@ -110,7 +116,7 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
   // (in runs of 256 columns of K, whatever the slab depth: the products of
   // a fused launch and of its halves then add in the same order)
   const int rot = (kRotates || a.rotate) && a.k >= 256
-                      ? tile % static_cast<int>(a.k / 256) * (256 / S::BK)
+                      ? tile / kXcds % static_cast<int>(a.k / 256) * (256 / S::BK)
                       : 0;
 
   // load instruction t of this wave: wave + 8 t of the slab's NI (weight
