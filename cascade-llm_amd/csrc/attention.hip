@@ -835,6 +835,180 @@ __attribute__((amdgpu_waves_per_eu(HW / 2))) void prefill_attention_kernel(
   if (half == 1) write_out();
 }
 
+// Short prompts.  The kernel above walks 32 tokens' positions in lockstep, a
+// barrier and about 2 us a 32-position step, and its workgroups number
+// tokens / 64 x KV heads: up to some hundred tokens most CUs idle through a
+// serial chain.  Here a workgroup owns 8 tokens of a KV head (two blocks of 16
+// MFMA columns) and its kShortWaves waves deal the 32-position blocks among
+// themselves, each with its own online softmax, fragments loaded straight to
+// registers as in the decode kernel (V transposed by byte permutes) and no
+// barrier until the waves' states merge in LDS.  Every block is read once per
+// 8 tokens instead of 32, from the L2 of the XCD that serves the KV head, so
+// past kShortTokens the traffic outweighs the shorter chain.  Against the
+// kernel above, from position 0: 6 tokens 5.8 -> 4.5 us, 45 10.6 -> 4.9, 157
+// 14.2 -> 6.6, 300 17.4 -> 8.8, 613 23.7 -> 20.3, 800 26.3 -> 26.8; after 4000
+// cached positions: 64 tokens 167 -> 44, 600 161 -> 137.  8 waves a
+// workgroup, and the next block's loads ahead of this one's products (two
+// register sets), were 5-10% slower.
+constexpr int kShortWaves = 4;
+constexpr int kShortTile = 8;
+constexpr int64_t kShortTokens = 704;
+constexpr int kShortPitch = kAttnD + 4;  // floats per column of a merged block
+
+__global__ __launch_bounds__(kShortWaves *kWave) void prefill_short_kernel(PrefillArgs a) {
+  constexpr int G = kAttnG, D = kAttnD, NB = 2;
+  __shared__ __attribute__((aligned(16))) float s_o[kShortWaves][16][kShortPitch];
+  __shared__ float s_ml[kShortWaves][NB][16][2];
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  // the longest walks first; a KV head's workgroups share an XCD when their
+  // count is a multiple of 8
+  const int g = static_cast<int>(blockIdx.x) % a.kv_heads;
+  const int unit = a.units - 1 - static_cast<int>(blockIdx.x) / a.kv_heads;
+  const int c16 = lane & 15;
+  const int g4 = lane >> 4;
+  const float c = a.scale_log2;
+  const int t0 = unit * kShortTile;
+  const int last_row = a.past + min(t0 + kShortTile, a.tokens) - 1;
+  const int blocks = last_row / kAttnBlock + 1;
+  const uint16_t *kb = a.k + g * a.head_stride;
+  const uint16_t *vb = a.v + g * a.head_stride;
+  const int krow = 8 * (c16 >> 2) + (c16 & 3);  // + 4 hf
+
+  // column c16 of block b: token t0 + 4 b + c16 / 4, query head 4 g + c16 % 4
+  u32x4 qop[NB][4];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const int t = min(t0 + 4 * b + (c16 >> 2), a.tokens - 1);
+    const uint16_t *qrow = a.q + static_cast<int64_t>(t) * a.q_row + (g * G + (c16 & 3)) * D;
+#pragma unroll
+    for (int cc = 0; cc < 4; ++cc)
+      qop[b][cc] = *reinterpret_cast<const u32x4 *>(qrow + 32 * cc + 8 * g4);
+  }
+  float m[NB], l[NB];
+  f32x4 o[NB][8];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    m[b] = -FLT_MAX;  // finite: a column with no valid row yet keeps alpha = 1
+    l[b] = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[b][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  for (int blk = wave; blk < blocks; blk += kShortWaves) {
+    const int r0 = blk * kAttnBlock;
+    u32x4 kt[2][4], vt[8];
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      const int row = min(r0 + krow + 4 * hf, last_row);
+#pragma unroll
+      for (int cc = 0; cc < 4; ++cc)
+        kt[hf][cc] = kv_load<false>(kb + static_cast<int64_t>(row) * D + 32 * cc + 8 * g4);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int row = min(r0 + 8 * g4 + j, last_row);
+      vt[j] = kv_load<false>(vb + static_cast<int64_t>(row) * D + 8 * c16);
+    }
+    const bool edge = r0 + kAttnBlock - 1 > a.past + t0;  // some column ends inside
+    u32x4 pop[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0;
+#pragma unroll
+      for (int cc = 0; cc < 4; ++cc) {
+        s0 = mfma_16x16x32_bf16(kt[0][cc], qop[b][cc], s0);
+        s1 = mfma_16x16x32_bf16(kt[1][cc], qop[b][cc], s1);
+      }
+      // s[j]: row r0 + 8 g4 + j, column c16 of block b
+      float s[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
+      if (edge) {
+        const int limit = a.past + t0 + 4 * b + (c16 >> 2);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (r0 + 8 * g4 + j > limit) s[j] = -INFINITY;
+      }
+      float bmax = max_f32(max_f32(max_f32(s[0], s[1]), max_f32(s[2], s[3])),
+                           max_f32(max_f32(s[4], s[5]), max_f32(s[6], s[7])));
+      bmax = xor32_max(xor16_max(bmax)) * c;
+      if (bmax > m[b] + kLazyRescale) {
+        const float alpha = exp2_fast(m[b] - bmax);
+        m[b] = bmax;
+        l[b] *= alpha;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[b][e] *= alpha;
+      }
+      const float nm = -m[b];
+      float p[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) p[j] = exp2_fast(fmaf(s[j], c, nm));
+      // P enters the MFMA rounded to bf16; l sums the fp32 values
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        pop[b][i] = pack_bf16x2(p[2 * i], p[2 * i + 1]);
+        l[b] += p[2 * i] + p[2 * i + 1];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const u32x4 ve = v_operand(vt, e);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) o[b][e] = mfma_16x16x32_bf16(ve, pop[b], o[b][e]);
+    }
+  }
+
+  // merge the waves, one column block at a time: o[b][e][r] = O[dim
+  // 8 (4 g4 + r) + e][column c16]
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    l[b] = xor32_sum(xor16_sum(l[b]));
+    if (g4 == 0) {
+      s_ml[wave][b][c16][0] = m[b];
+      s_ml[wave][b][c16][1] = l[b];
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    if (b) __syncthreads();  // block b - 1 is read
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        *reinterpret_cast<f32x4 *>(&s_o[wave][c16][8 * (4 * g4 + r) + 4 * h]) =
+            f32x4{o[b][4 * h][r], o[b][4 * h + 1][r], o[b][4 * h + 2][r], o[b][4 * h + 3][r]};
+    __syncthreads();
+    // thread: kDims consecutive dims of a column
+    constexpr int kDims = 16 * D / (kShortWaves * kWave);
+    const int col = tid / (D / kDims), d0 = kDims * (tid % (D / kDims));
+    const int t = t0 + 4 * b + col / 4;
+    if (t < a.tokens) {
+      float mx = s_ml[0][b][col][0];
+#pragma unroll
+      for (int w = 1; w < kShortWaves; ++w) mx = fmaxf(mx, s_ml[w][b][col][0]);
+      float den = 0.0f;
+      f32x4 sum[kDims / 4];
+#pragma unroll
+      for (int q = 0; q < kDims / 4; ++q) sum[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int w = 0; w < kShortWaves; ++w) {
+        const float wt = exp2_fast(s_ml[w][b][col][0] - mx);
+        den = fmaf(wt, s_ml[w][b][col][1], den);
+#pragma unroll
+        for (int q = 0; q < kDims / 4; ++q)
+          sum[q] += *reinterpret_cast<const f32x4 *>(&s_o[w][col][d0 + 4 * q]) * wt;
+      }
+      const float inv = 1.0f / den;
+      uint16_t *dst = a.out + static_cast<int64_t>(t) * a.q_row + (g * G + col % 4) * D + d0;
+#pragma unroll
+      for (int q = 0; q < kDims / 4; ++q)
+        *reinterpret_cast<uint2 *>(dst + 4 * q) =
+            uint2{pack_bf16x2(sum[q][0] * inv, sum[q][1] * inv),
+                  pack_bf16x2(sum[q][2] * inv, sum[q][3] * inv)};
+    }
+  }
+}
+
+
 constexpr size_t attention_workspace(int64_t nsplits, int64_t n_kv_heads) {
   const size_t per = static_cast<size_t>(n_kv_heads) * nsplits * kAttnG;
   return kAttnHeaderBytes + per * 2 * sizeof(float) +
@@ -1085,10 +1259,15 @@ extern "C" int cascade_prefill_attention_bf16(
   a.past = static_cast<int32_t>(past);
   a.tokens = static_cast<int32_t>(tokens);
   a.q_row = static_cast<int32_t>(n_q_heads * head_dim);
-  a.units = static_cast<int32_t>((tokens + kPrefillUnit - 1) / kPrefillUnit);
+  const int tile = tokens <= kShortTokens ? kShortTile : kPrefillUnit;
+  a.units = static_cast<int32_t>((tokens + tile - 1) / tile);
   a.kv_heads = static_cast<int32_t>(n_kv_heads);
   a.scale_log2 = scale * kLog2e;
   a.out = static_cast<uint16_t *>(out);
+  if (tokens <= kShortTokens)
+    return launch_kernel(prefill_short_kernel,
+                         dim3(static_cast<unsigned>(a.units * n_kv_heads)),
+                         dim3(kShortWaves * kWave), 0, static_cast<hipStream_t>(stream), a);
   // one workgroup per (unit pair, KV head); consecutive workgroups take
   // consecutive KV heads
   const int64_t workgroups = (a.units + 1) / 2 * n_kv_heads;
