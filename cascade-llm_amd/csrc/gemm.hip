@@ -9,14 +9,13 @@
 // resident LM head, llama31.py:330-334).
 //
 // Tiling.  A workgroup computes a BM x 128 output tile (or two side by
-// side), K walked in 64-deep slabs (32-deep for the 256-column tiles); each
+// side), K walked in 64-deep slabs; each
 // wave owns 64 (or 128) rows x 64 (or 32) columns of
 // v_mfma_f32_16x16x32_bf16 fragments and reads its A and B fragments (16
 // bytes a lane) from LDS.  Shapes (launch_gemm picks one):
 //   GemmTileWide 256 x 256 (two 128-column sub-tiles), 8 waves of 128 x 64,
-//                32-deep slabs on a ring of 4: where its schedule of rounds
-//                is shorter than GemmTile256's (the resident LM head over
-//                every prompt row at M = 2048: 16 rounds);
+//                64-deep slabs in two buffers (gemm_wide_run): where its
+//                schedule of rounds is shorter than GemmTile256's;
 //   GemmTile256  256 x 128, 8 waves, a ring of 3 slab buffers: the large
 //                GEMMs (at least as many 256-row tiles as CUs: q, o, gate,
 //                up, down and the fused gate|up at M = 2048);
@@ -50,8 +49,7 @@
 // N = 6144 95.8 -> 85.2, fused gate|up 407.0 -> 395.1).
 //
 // LDS layout of a slab: 128-byte rows (64 bf16) back to back; 16-byte
-// chunk c of row r sits at chunk c ^ ((r / 2) % 8) (32-deep slabs: 64-byte
-// rows, chunk c ^ ((r / 4) % 4)).  A fragment read (16
+// chunk c of row r sits at chunk c ^ ((r / 2) % 8).  A fragment read (16
 // lanes: 16 consecutive rows, one chunk) then hits 16 distinct 16-byte bank
 // groups, each read is a per-lane base plus an immediate offset, and a load
 // instruction (64 lanes x 16 bytes) fills 8 whole rows, so its lanes read
@@ -441,6 +439,18 @@ struct GemmRing {
   static constexpr int LDS = STAGES * SLAB > STAGE ? STAGES * SLAB : STAGE;
 };
 
+// The matrix of q|k|v head h, its rows and the head's first row in it.
+struct HeadRows {
+  const uint16_t *base;
+  int64_t rows, row;
+};
+__device__ __forceinline__ HeadRows head_rows(const GemmArgs &a, int64_t h) {
+  const int64_t hq = a.n0 / kGemmHead, hk = a.n1 / kGemmHead;
+  if (h < hq) return {a.w0, a.n0, h * kGemmHead};
+  if (h < hq + hk) return {a.w1, a.n1, (h - hq) * kGemmHead};
+  return {a.w2, a.n2, (h - hq - hk) * kGemmHead};
+}
+
 // Output tile (tm, tn) of shape T: rows tm * BM .., 128-column sub-tiles
 // tn * NSUB .. (q|k|v: head tn; SwiGLU: gate / up rows 64 per sub-tile).
 // sb0 holds the ring.
@@ -448,7 +458,6 @@ template <int EPI, class T, int STAGES, int BK = kTileK>
 __device__ __forceinline__ void gemm_tile_run(const GemmArgs &a, int tm, int tn,
                                               uint16_t *sb0) {
   static_assert(STAGES >= 3, "a ring of at least 3 slab buffers");
-  static_assert(T::NSUB == 1 || EPI != kGemmQkvRope, "q|k|v: one head per tile");
   using L = DmaSlab<BK>;
   using R = GemmRing<T, STAGES, BK>;
   constexpr int XI = T::BM * L::ROWB / 1024;  // load instructions per X slab
@@ -474,15 +483,11 @@ __device__ __forceinline__ void gemm_tile_run(const GemmArgs &a, int tm, int tn,
     wbase0 = a.w0; wrows0 = a.n0; wrow0 = static_cast<int64_t>(tn) * T::NSUB * kGemmHalfHead;
     wbase1 = a.w1; wrows1 = a.n0; wrow1 = wrow0;
   } else if constexpr (EPI == kGemmQkvRope) {
-    const int64_t hq = a.n0 / kGemmHead, hk = a.n1 / kGemmHead;
-    if (tn < hq) {
-      wbase0 = a.w0; wrows0 = a.n0; wrow0 = static_cast<int64_t>(tn) * kGemmHead;
-    } else if (tn < hq + hk) {
-      wbase0 = a.w1; wrows0 = a.n1; wrow0 = (tn - hq) * kGemmHead;
-    } else {
-      wbase0 = a.w2; wrows0 = a.n2; wrow0 = (tn - hq - hk) * kGemmHead;
-    }
-    wbase1 = wbase0; wrows1 = wrows0; wrow1 = wrow0;
+    // one head per sub-tile
+    const HeadRows h0 = head_rows(a, static_cast<int64_t>(tn) * T::NSUB);
+    const HeadRows h1 = head_rows(a, static_cast<int64_t>(tn) * T::NSUB + T::NSUB - 1);
+    wbase0 = h0.base; wrows0 = h0.rows; wrow0 = h0.row;
+    wbase1 = h1.base; wrows1 = h1.rows; wrow1 = h1.row;
   } else {
     wbase0 = a.w0; wrows0 = a.n0; wrow0 = static_cast<int64_t>(tn) * T::BN;
     wbase1 = wbase0; wrows1 = wrows0; wrow1 = wrow0;
@@ -539,11 +544,14 @@ __device__ __forceinline__ void gemm_tile_run(const GemmArgs &a, int tm, int tn,
       const int trow = L::RPI * i;  // tile row of the instruction
       // SwiGLU: sub-tile trow / 128 holds 64 gate rows, then their 64 up rows
       const int tt = trow % kTileN;
-      const bool second = EPI == kGemmSwiglu && tt >= kGemmHalfHead;
+      const bool second = EPI == kGemmSwiglu    ? tt >= kGemmHalfHead
+                          : EPI == kGemmQkvRope ? trow >= kTileN
+                                                : false;
       const int64_t row =
           EPI == kGemmSwiglu
               ? (second ? wrow1 : wrow0) + (trow / kTileN) * kGemmHalfHead + tt % kGemmHalfHead
-              : wrow0 + trow;
+          : EPI == kGemmQkvRope ? (second ? wrow1 : wrow0) + tt
+                                : wrow0 + trow;
       dma_lds16(second ? ww1 : ww0,
                 ((i & 1) ? ld_off1 : ld_off0) + static_cast<int>(row * k_bytes) + kb,
                 dw + i * 1024);
@@ -676,6 +684,205 @@ __device__ __forceinline__ void gemm_tile_run(const GemmArgs &a, int tm, int tn,
   }
 }
 
+// The same for a 256 x 256 tile (GemmTileWide): 64-deep slabs, so that a
+// load instruction reads 128-byte row segments, in two buffers.  Three slabs
+// of 64 KiB do not fit the LDS, and 32-deep ones, which did, read 64-byte
+// segments: the load path then moves 46 GB/s a CU where 128-byte and longer
+// ones reach 59 (256 x 256 tiles' loads alone, 32 CUs of an XCD on 4 x 8
+// tiles; ring depths 3 to 5 alike), and the loads took longer than the
+// products.  A slab comes in four units of 128 rows: A0, A1 (each wave row's
+// first and last 64 of its 128 rows) and B0, B1 (fragment columns j < 2 and
+// j >= 2).  Its 64 products a wave take two steps:
+//   step 2s      A0 x B0, A0 x B1   while B1 and A1 of slab s are read
+//   step 2s + 1  A1 x B1, A1 x B0   while A0 and B0 of slab s + 1 are read
+// Each step opens with a wait and a barrier, which publish the units it
+// reads and free those the step before read; these take the same units of
+// slab s + 2: A0, B0 in step 2s, B1, A1 in step 2s + 1.  So every load has
+// three steps to land (4 instructions a wave and step, 8 in flight past each
+// wait) and two buffers hold what three would.  B0 of slab s + 1 is read
+// over B1's registers: the two B register sets swap roles from slab to slab.
+// K is added in the order of every other tile, bit for bit.
+template <int EPI>
+__device__ __forceinline__ void gemm_wide_run(const GemmArgs &a, int tm, int tn, uint16_t *sb0) {
+  using T = GemmTileWide;
+  constexpr int BK = kTileK;
+  using L = DmaSlab<BK>;
+  static_assert(T::FM == 8 && T::FN == 4 && T::BM == 256 && T::BN == 256, "unit geometry");
+  constexpr int XB = T::BM * BK, kSlab = (T::BM + T::BN) * BK;  // bf16 elements
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int sub = wave / T::SUBWAVES;
+  const int sw = wave % T::SUBWAVES;
+  const int wm = sw / T::WN;
+  const int wn = sw % T::WN;
+  const int lr = lane & 15;
+  const int g4 = lane >> 4;
+  const int64_t k_bytes = a.k * 2;
+  const u32x4 xw = buffer_rsrc_words(a.x, a.m * k_bytes);
+  // the matrices of the tile's weight rows and its first row in each: gate
+  // and up (SwiGLU), or of each sub-tile's head (q|k|v)
+  u32x4 ww0, ww1;
+  int64_t wrow0, wrow1;
+  if constexpr (EPI == kGemmQkvRope) {
+    const HeadRows h0 = head_rows(a, static_cast<int64_t>(tn) * 2);
+    const HeadRows h1 = head_rows(a, static_cast<int64_t>(tn) * 2 + 1);
+    ww0 = buffer_rsrc_words(h0.base, h0.rows * k_bytes);
+    ww1 = buffer_rsrc_words(h1.base, h1.rows * k_bytes);
+    wrow0 = h0.row;
+    wrow1 = h1.row;
+  } else {
+    ww0 = buffer_rsrc_words(a.w0, a.n0 * k_bytes);
+    ww1 = buffer_rsrc_words(EPI == kGemmSwiglu ? a.w1 : a.w0, a.n0 * k_bytes);
+    wrow0 = wrow1 =
+        static_cast<int64_t>(tn) * (EPI == kGemmSwiglu ? T::NSUB * kGemmHalfHead : T::BN);
+  }
+
+  // load instruction i (0 .. 15) of a unit fills its 8 rows 8 i ..; the
+  // wave issues i = 2 wave + e, whose parity is e
+  const int ld_r = lane / L::CH;
+  int ld_off[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int f = ((L::RPI * e + ld_r) / L::RPB) % L::CH;
+    ld_off[e] = ld_r * static_cast<int>(k_bytes) + 16 * ((lane % L::CH) ^ f);
+  }
+  const int fl = (lr / L::RPB) % L::CH;
+  const int rd_off0 = lr * L::ROWB + 16 * (g4 ^ fl);
+  const int rd_off1 = lr * L::ROWB + 16 * ((4 + g4) ^ fl);
+  const int slabs = static_cast<int>(a.k / BK);
+  const uint32_t ring_lds = lds_address(sb0);
+
+  // row of the tile's 256 that row r (0 .. 127) of half `half` is
+  auto unit_row = [](int r, int half) { return r % 64 + 128 * (r / 64) + 64 * half; };
+  // h 0, 1: this wave's instructions of unit A<half>; 2, 3: of unit B<half>
+  auto load_one = [&](int slab, int buf, int half, int h) __attribute__((always_inline)) {
+    const int e = h & 1;
+    const int trow = unit_row(L::RPI * (2 * wave + e), half);
+    const int kb = slab * BK * 2;
+    const uint32_t dst = ring_lds + static_cast<uint32_t>(buf * kSlab * 2 + trow * L::ROWB);
+    if (h < 2) {
+      const int64_t row = static_cast<int64_t>(tm) * T::BM + trow;
+      dma_lds16(xw, ld_off[e] + static_cast<int>(row * k_bytes) + kb, dst);
+    } else {
+      // SwiGLU: sub-tile trow / 128 holds 64 gate rows (B0), 64 up rows (B1)
+      const int64_t row =
+          EPI == kGemmSwiglu
+              ? wrow0 + (trow / kTileN) * kGemmHalfHead + trow % kGemmHalfHead
+          : EPI == kGemmQkvRope ? (trow >= kTileN ? wrow1 : wrow0) + trow % kTileN
+                                : wrow0 + trow;
+      const bool second = EPI == kGemmQkvRope ? trow >= kTileN : half == 1;
+      dma_lds16(second ? ww1 : ww0, ld_off[e] + static_cast<int>(row * k_bytes) + kb,
+                dst + XB * 2);
+    }
+  };
+
+  f32x4 acc[T::FM][T::FN];
+#pragma unroll
+  for (int i = 0; i < T::FM; ++i)
+#pragma unroll
+    for (int j = 0; j < T::FN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  using Quad = u32x4[2][4];  // [32-deep half][fragment] of an A unit
+  using Pair = u32x4[2][2];  // of a B unit
+  Quad fa0, fa1;
+  Pair fb0, fb1;
+  auto read_a = [&](int buf, int half, int r, Quad &f) __attribute__((always_inline)) {
+    const int ks = r / 4, i = r % 4;
+    f[ks][i] = *reinterpret_cast<const u32x4 *>(
+        reinterpret_cast<const char *>(sb0 + buf * kSlab) + (ks ? rd_off1 : rd_off0) +
+        (128 * wm + 64 * half + 16 * i) * L::ROWB);
+  };
+  auto read_b = [&](int buf, int half, int r, Pair &f) __attribute__((always_inline)) {
+    const int ks = r / 2, j = r % 2;
+    f[ks][j] = *reinterpret_cast<const u32x4 *>(
+        reinterpret_cast<const char *>(sb0 + buf * kSlab + XB) + (ks ? rd_off1 : rd_off0) +
+        (kTileN * sub + gemm_col<T>(wn, 2 * half + j, lr) - lr) * L::ROWB);
+  };
+  constexpr int kWaitStep = waitcnt_imm(8, 0);
+  // One step: the 32 products of A unit `ha` (fragments `a_frag`) with B unit
+  // `hb` (`b_first`), then with the other one (`b_second`), in 4 chunks of a
+  // load instruction, 8 products and 3 fragment reads; loads(h) issues load
+  // h, reads(r) makes fragment read r (0 .. 11).
+  auto step = [&](const Quad &fa, int ha, const Pair &b_first, int hb, const Pair &b_second,
+                  auto loads, auto reads) __attribute__((always_inline)) {
+    auto product = [&](int idx) __attribute__((always_inline)) {
+      const int half = idx / 16, ks = (idx / 8) % 2, i = (idx / 2) % 4, j = idx % 2;
+      const int col = 2 * (half ? 1 - hb : hb) + j;
+      const u32x4 b = half ? b_second[ks][j] : b_first[ks][j];
+      acc[4 * ha + i][col] = mfma_16x16x32_bf16(fa[ks][i], b, acc[4 * ha + i][col]);
+    };
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(kWaitStep);
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int idx = 0; idx < 4; ++idx) product(idx);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      loads(c);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int idx = 4 + 7 * c; idx < 11 + 7 * c; ++idx) product(idx);
+#pragma unroll
+      for (int r = 3 * c; r < 3 * c + 3; ++r) reads(r);
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // both steps of a slab in buffer buf; b0 holds its B0 fragments on entry,
+  // b1 those of slab s + 1 on return
+  auto slab_steps = [&](int s, int buf, Pair &b0, Pair &b1) __attribute__((always_inline)) {
+    const int next = min(s + 2, slabs - 1);
+    step(fa0, 0, b0, 0, b1,
+         [&](int h) __attribute__((always_inline)) { load_one(next, buf, 0, h); },
+         [&](int r) __attribute__((always_inline)) {
+           if (r < 4) read_b(buf, 1, r, b1);
+           else read_a(buf, 1, r - 4, fa1);
+         });
+    step(fa1, 1, b1, 1, b0,
+         [&](int h) __attribute__((always_inline)) { load_one(next, buf, 1, h); },
+         [&](int r) __attribute__((always_inline)) {
+           if (r < 8) read_a(1 - buf, 0, r, fa0);
+           else read_b(1 - buf, 0, r - 8, b1);
+         });
+  };
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+      for (int h = 0; h < 4; ++h) load_one(min(p, slabs - 1), p, half, h);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(waitcnt_imm(12, 0));
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int r = 0; r < 8; ++r) read_a(0, 0, r, fa0);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) read_b(0, 0, r, fb0);
+  int s = 0;
+  for (; s + 2 <= slabs; s += 2) {
+    slab_steps(s, 0, fb0, fb1);
+    slab_steps(s + 1, 1, fb1, fb0);
+  }
+  if (s < slabs) slab_steps(s, 0, fb0, fb1);
+  // every load landed and every LDS read done before the ring is reused
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
+  if (EPI != kGemmF32 && a.vec_out) {
+    __builtin_amdgcn_s_barrier();
+    gemm_epilogue_staged<EPI, T>(a, tm, tn * T::NSUB + sub, wm, wn, lane, sw, acc,
+                                 sb0 + sub * (kTileN * T::STAGE_COL));
+  } else {
+    gemm_epilogue<EPI, T>(a, tm, tn * T::NSUB + sub, wm, wn, lane, acc);
+  }
+}
+
 // One launch covers the output with tiles of shape T and, when the last
 // round of T tiles would leave at least half of the CUs idle, the last
 // tail_n tile columns with tiles of half the height (TH, the same wave
@@ -702,7 +909,10 @@ __global__ __launch_bounds__(T::WAVES *kWave) void gemm_kernel(GemmArgs a) {
   // padding workgroups leave as a whole: no barrier is skipped
   if (j < a.per_xcd) {
     if (!gemm_tile(xcd * a.per_xcd + j, a.tiles, a.tiles_m, a.tiles_n, tm, tn)) return;
-    gemm_tile_run<EPI, T, STAGES, BK>(a, tm, tn, sb0);
+    if constexpr (std::is_same<T, GemmTileWide>::value)
+      gemm_wide_run<EPI>(a, tm, tn, sb0);
+    else
+      gemm_tile_run<EPI, T, STAGES, BK>(a, tm, tn, sb0);
     return;
   }
   if constexpr (!std::is_same<T, TH>::value) {
@@ -808,33 +1018,30 @@ static hipError_t launch_gemm(GemmArgs &a, int64_t tiles_n, hipStream_t s) {
   if (sp.fm) return launch_stream(EPI, sp, a, s);
   const int64_t tiles256 = (a.m + 255) / 256 * tiles_n;
   if (a.m > 128 && tiles256 >= cus) {
-    // 256 x 256 tiles read a quarter less X and W per MFMA but need 32-deep
-    // slabs (a ring of four 32 KiB slabs; 64-deep ones would not fit three
-    // in the LDS), so twice the step barriers.  The schedule of rounds
-    // decides, with round costs measured at M = 2048, K = 4096 (in rounds
-    // of 256 x 128 tiles, about 58 us each): a round of 256 x 256 tiles
-    // 1.98 (N = 16384: 230 us for 2 rounds against 244 us for 4), a round of
-    // their 128 x 256 half-height tail tiles 1.2, a round of 128 x 128 tail
-    // tiles 0.7.  So the fused gate|up (N = 2 x 14336) runs 7 rounds of
-    // 256 x 128 tiles (405.8 us) rather than 3 rounds + a half-height round
-    // of 256 x 256 (414.5 us), and the resident LM head (N = 128256) 16
-    // rounds of 256 x 256 (1712 against 1784 us).  SwiGLU needs whole
-    // pairs of 128-column gate / up groups; q|k|v keeps one head per tile.
-    if constexpr (EPI != kGemmQkvRope) {
-      const int64_t tm256 = (a.m + 255) / 256, tm128 = (a.m + 127) / 128;
-      const int64_t wide_n = (tiles_n + 1) / 2;
-      const TileRounds std_r = tile_rounds(tm256, tiles_n, tm128, cus);
-      const TileRounds wide_r = tile_rounds(tm256, wide_n, tm128, cus);
-      constexpr double kWideRound = 1.98;  // in rounds of 256 x 128 tiles
-      constexpr double kWideHalfRound = 1.2;
-      constexpr double kHalfRound = 0.7;
-      const double std_t = static_cast<double>(std_r.full) +
-                           (std_r.tail == 1 ? kHalfRound : std_r.tail == 2 ? 1.0 : 0.0);
-      const double wide_t = kWideRound * static_cast<double>(wide_r.full) +
-                            (wide_r.tail == 1 ? kWideHalfRound : wide_r.tail == 2 ? kWideRound : 0.0);
-      if (wide_t < std_t && (EPI != kGemmSwiglu || tiles_n % 2 == 0))
-        return launch_tiles<EPI, 32, GemmTileWide, 4, GemmTileWideHalf, 4>(a, wide_n, cus, s);
-    }
+    // 256 x 256 tiles read a third less X and W per product, which is what
+    // bounds these launches.  The schedule of rounds decides, with round
+    // costs measured at M = 2048 and 8192, K = 4096 (in rounds of 256 x 128
+    // tiles, about 57 us each): a round of 256 x 256 tiles 1.7 (97 us), a
+    // round of their 128 x 256 half-height tail tiles 1.15, a round of
+    // 128 x 128 tail tiles 0.7.  So the fused gate|up (N = 2 x 14336) at
+    // M = 2048 runs 3 rounds + a half-height round of 256 x 256 (358 us)
+    // rather than 7 rounds of 256 x 128 tiles (400 us); o_proj and q keep
+    // their one round of 256 x 128 (57 us).  SwiGLU and q|k|v need whole
+    // pairs of 128-column gate / up groups or heads.
+    const int64_t tm256 = (a.m + 255) / 256, tm128 = (a.m + 127) / 128;
+    const int64_t wide_n = (tiles_n + 1) / 2;
+    const TileRounds std_r = tile_rounds(tm256, tiles_n, tm128, cus);
+    const TileRounds wide_r = tile_rounds(tm256, wide_n, tm128, cus);
+    constexpr double kWideRound = 1.7;  // in rounds of 256 x 128 tiles
+    constexpr double kWideHalfRound = 1.15;
+    constexpr double kHalfRound = 0.7;
+    const double std_t = static_cast<double>(std_r.full) +
+                         (std_r.tail == 1 ? kHalfRound : std_r.tail == 2 ? 1.0 : 0.0);
+    const double wide_t = kWideRound * static_cast<double>(wide_r.full) +
+                          (wide_r.tail == 1 ? kWideHalfRound : wide_r.tail == 2 ? kWideRound : 0.0);
+    constexpr bool kWholePairs = EPI == kGemmSwiglu || EPI == kGemmQkvRope;
+    if (wide_t < std_t && (!kWholePairs || tiles_n % 2 == 0))
+      return launch_tiles<EPI, kTileK, GemmTileWide, 2, GemmTileWideHalf, 3>(a, wide_n, cus, s);
     return launch_tiles<EPI, kTileK, GemmTile256, 3, GemmTile128x8, 4>(a, tiles_n, cus, s);
   }
   const int64_t tiles128 = (a.m + 127) / 128 * tiles_n;
