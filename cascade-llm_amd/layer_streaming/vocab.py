@@ -138,6 +138,7 @@ class VocabStreamingRuntime:
         self._free = [_hip.HipEvent() for _ in range(chunks)]
         self._staging_read = [None, None]  # copy that last read a pinned half
         self._prestaged = {}  # chunk -> future of its staged pinned half
+        self._deferred = set()  # chunks whose half was not free to stage into
         self._start = _hip.HipEvent()
         # gather groups alternate between the two halves of the row buffer
         # (one group of its single row when it holds one)
@@ -215,8 +216,15 @@ class VocabStreamingRuntime:
 
         if chunk >= self.vocab.chunk_count or chunk in self._prestaged:
             return
-        rows = self._chunk_rows(chunk)
         half = chunk % 2
+        if any(c % 2 == half for c in self._prestaged):
+            # the half holds a chunk that is not copied yet: a model of few
+            # units has its next call staged whole, and so asks for that
+            # call's first chunks, while this call's last ones still wait
+            self._deferred.add(chunk)
+            return
+        self._deferred.discard(chunk)
+        rows = self._chunk_rows(chunk)
         reader = self._staging_read[half]
         target = self.head_staging_slots[half][: rows.numel()]
         self._prestaged[chunk] = self.store.stage_into(
@@ -252,6 +260,7 @@ class VocabStreamingRuntime:
             except Exception:  # the call that queued it already raised
                 pass
         self._prestaged = {}
+        self._deferred = set()
 
     def _copy_chunk(self, chunk):
         first, end = self.vocab.chunk_bounds(chunk)
@@ -269,6 +278,8 @@ class VocabStreamingRuntime:
             # is staged there once it is done
             self._staging_read[chunk % 2] = self._ready[chunk]
             self._prestage(chunk + 2)
+            if chunk % 2 in self._deferred:
+                self._prestage(chunk % 2)
 
     def _copy_first_chunk(self, slot):
         """Release hook of the transformer runtime: its last unit in

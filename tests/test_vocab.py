@@ -203,3 +203,49 @@ def test_release_hook_holds_the_vocabulary_runtime_weakly(monkeypatch):
             gc.enable()
     assert runtime.release_hook(0) is False
     assert released == [1]
+
+
+@pytest.mark.parametrize("chunks", [4, 5, 8])
+def test_staged_halves_are_copied_before_they_are_filled_again(chunks):
+    # A model whose units all stage ahead of the next call asks for that
+    # call's first chunks while this call's last two still wait in the
+    # pinned halves: a half is filled again only once its chunk is copied.
+    from types import SimpleNamespace
+
+    from layer_streaming.vocab import VocabStreamingRuntime
+
+    vocab = VocabStreamingRuntime.__new__(VocabStreamingRuntime)
+    holds, copied = [None, None], []
+
+    def stage_into(target, source, waits):
+        half, chunk = target[0].item(), int(source[0])
+        assert holds[half] is None, "chunk {} over chunk {}".format(chunk, holds[half])
+        # it waits for the copy that last read the half
+        last = [c for c in copied if c % 2 == half][-1:]
+        assert list(waits) == ["ready {}".format(c) for c in last]
+        holds[half] = chunk
+        return SimpleNamespace(result=lambda: chunk)
+
+    def slot_copy(slot, kind, chunk, source, nbytes, ready, pair):
+        assert source == chunk == holds[slot]
+        holds[slot] = None
+        copied.append(chunk)
+
+    vocab.vocab = SimpleNamespace(chunk_count=chunks, hidden_size=1,
+                                  chunk_bounds=lambda c: (c, c + 1),
+                                  lm_head_key="head")
+    vocab.store = SimpleNamespace(
+        tensor=lambda key: torch.arange(chunks).view(-1, 1), stage_into=stage_into)
+    vocab.transformer_runtime = SimpleNamespace(
+        slot_copy=slot_copy, stage_call_ahead=vocab._prestage_first_chunks)
+    vocab.head_staging_slots = [torch.tensor([0]), torch.tensor([1])]
+    vocab.profile, vocab._staged = False, True
+    vocab._ready = ["ready {}".format(c) for c in range(chunks)]
+    vocab._staging_read, vocab._prestaged, vocab._deferred = [None, None], {}, set()
+    for _ in range(3):
+        first = len(copied)
+        for chunk in range(chunks):
+            vocab._copy_chunk(chunk)
+        assert copied[first:] == list(range(chunks))
+    # the next call's first chunks are staged behind the last copies
+    assert [h for h in holds if h is not None] == list(range(min(2, chunks)))
