@@ -16,6 +16,10 @@
 //   GemmTileWide 256 x 256 (two 128-column sub-tiles), 8 waves of 128 x 64,
 //                64-deep slabs in two buffers (gemm_wide_run): where its
 //                schedule of rounds is shorter than GemmTile256's;
+//   GemmTile160  160 x 256 (two sub-tiles), 8 waves of 80 x 64, a ring of 3:
+//                prompts that fill 160-row tiles better than 256-row ones
+//                (129 .. 160, 257 .. 320, 513 .. 640 rows), and split K
+//                where its tiles divide over the CUs more evenly;
 //   GemmTile256  256 x 128, 8 waves, a ring of 3 slab buffers: the large
 //                GEMMs (at least as many 256-row tiles as CUs: q, o, gate,
 //                up, down and the fused gate|up at M = 2048);
@@ -137,6 +141,7 @@ using GemmTile64 = GemmTile<64, 1, 4>;    // 4 waves of 64 x 32
 using GemmTile128x8 = GemmTile<128, 2, 4>;  // 8 waves of 64 x 32 (half of GemmTile256)
 using GemmTileWide = GemmTile<256, 2, 2, 2>;      // 8 waves of 128 x 64, 256 columns
 using GemmTileWideHalf = GemmTile<128, 2, 2, 2>;  // 8 waves of 64 x 64, 256 columns
+using GemmTile160 = GemmTile<160, 2, 2, 2>;       // 8 waves of 80 x 64, 256 columns
 
 // Tile column of fragment j of wave column wn for lane row lr.  A wave's
 // first-half fragments (j < H) and second-half fragments (j >= H) sit 64
@@ -462,12 +467,16 @@ __device__ __forceinline__ void gemm_tile_run(const GemmArgs &a, int tm, int tn,
   using R = GemmRing<T, STAGES, BK>;
   constexpr int XI = T::BM * L::ROWB / 1024;  // load instructions per X slab
   constexpr int WI = T::BN * L::ROWB / 1024;
-  constexpr int XW = XI / T::WAVES, WW = WI / T::WAVES;  // per wave
-  static_assert(XI % T::WAVES == 0 && WI % T::WAVES == 0, "whole loads per wave");
+  // per wave; 160-row tiles leave waves XR .. 7 one X load fewer than the
+  // others (the last of the XW, and of every vmcnt below)
+  constexpr int XW = (XI + T::WAVES - 1) / T::WAVES, WW = WI / T::WAVES;
+  constexpr int XR = XI % T::WAVES;
+  static_assert(WI % T::WAVES == 0, "whole W loads per wave");
   constexpr int XB = R::XB, kSlab = R::SLAB;
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const bool more = XR == 0 || wave < XR;  // issues all XW of its X loads
   const int sub = wave / T::SUBWAVES;  // sub-tile of the wave
   const int sw = wave % T::SUBWAVES;
   const int wm = sw / T::WN;
@@ -535,7 +544,8 @@ __device__ __forceinline__ void gemm_tile_run(const GemmArgs &a, int tm, int tn,
     const uint32_t dw = dx + XB * 2;
     const int kb = (slab0 + slab) * BK * 2;
     if (h < XW) {
-      const int i = wave * XW + h;
+      if (h == XW - 1 && !more) return;
+      const int i = XR ? wave + T::WAVES * h : wave * XW + h;
       const int64_t row = static_cast<int64_t>(tm) * T::BM + L::RPI * i;
       dma_lds16(xw, ((i & 1) ? ld_off1 : ld_off0) + static_cast<int>(row * k_bytes) + kb,
                 dx + i * 1024);
@@ -578,8 +588,6 @@ __device__ __forceinline__ void gemm_tile_run(const GemmArgs &a, int tm, int tn,
   constexpr int kAhead = (STAGES - 2) * D;
   constexpr int kAheadFirst = (STAGES - 1) * D;
   static_assert(kAheadFirst < 64, "vmcnt holds 6 bits");
-  constexpr int kWaitStep = waitcnt_imm(kAhead, 0);
-  constexpr int kWaitFirst = waitcnt_imm(kAheadFirst, 0);
   constexpr int kWaitAll = waitcnt_imm(0, 0);
   constexpr int KS = BK / 32;
   constexpr int kReads = KS * (T::FM + T::FN);
@@ -612,7 +620,10 @@ __device__ __forceinline__ void gemm_tile_run(const GemmArgs &a, int tm, int tn,
   // asm pins memory accesses in program order)
   auto publish_step = [&]() {
     asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(kWaitStep);
+    if (more)
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm(kAhead, 0));
+    else
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm(kAhead - (STAGES - 2), 0));
     __builtin_amdgcn_s_barrier();
   };
   int cur = 0;  // buffer of slab s
@@ -661,7 +672,10 @@ __device__ __forceinline__ void gemm_tile_run(const GemmArgs &a, int tm, int tn,
   for (int p = 0; p < STAGES; ++p) ring_load(min(p, slabs - 1), p);
   FragA fa0, fa1;
   FragB fb0, fb1;
-  __builtin_amdgcn_s_waitcnt(kWaitFirst);
+  if (more)
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm(kAheadFirst, 0));
+  else
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm(kAheadFirst - (STAGES - 1), 0));
   __builtin_amdgcn_s_barrier();
 #pragma unroll
   for (int r = 0; r < kReads; ++r) read_frag(0, r, fa0, fb0);
@@ -989,6 +1003,14 @@ struct TileRounds {
   int64_t full;
   int tail;
 };
+// A round of 160 x 256 tiles, in rounds of 256 x 128 tiles of the same K
+// (K = 4096: 70 to 76 us).  A launch is bounded by what each CU's load path
+// moves (about 60 GB/s of X and W rows), so a round costs its rows of both,
+// and rows of padding cost as much as any: 160 rows waste fewer of them at
+// 129 .. 160 rows (logits of 157 rows 222 -> 209 us), 257 .. 320 (gate|up
+// 92.7 -> 76.0 at 320; logits 374 -> 313) and 513 .. 640 (gate|up of 613
+// rows 151.8 -> 139.2).  192-row tiles' ring of 3 would not fit the LDS.
+constexpr double kLowRound = 1.3;
 static TileRounds tile_rounds(int64_t tiles_m, int64_t tiles_n, int64_t htiles_m, int cus) {
   const int64_t tiles = tiles_m * tiles_n;
   const int64_t rem = tiles % cus;
@@ -1040,6 +1062,10 @@ static hipError_t launch_gemm(GemmArgs &a, int64_t tiles_n, hipStream_t s) {
     const double wide_t = kWideRound * static_cast<double>(wide_r.full) +
                           (wide_r.tail == 1 ? kWideHalfRound : wide_r.tail == 2 ? kWideRound : 0.0);
     constexpr bool kWholePairs = EPI == kGemmSwiglu || EPI == kGemmQkvRope;
+    const double low_t = kLowRound * static_cast<double>(
+        ((a.m + 159) / 160 * wide_n + cus - 1) / cus);
+    if (low_t < std::min(std_t, wide_t) && (!kWholePairs || tiles_n % 2 == 0))
+      return launch_tiles<EPI, kTileK, GemmTile160, 3>(a, wide_n, cus, s);
     if (wide_t < std_t && (!kWholePairs || tiles_n % 2 == 0))
       return launch_tiles<EPI, kTileK, GemmTileWide, 2, GemmTileWideHalf, 3>(a, wide_n, cus, s);
     return launch_tiles<EPI, kTileK, GemmTile256, 3, GemmTile128x8, 4>(a, tiles_n, cus, s);
@@ -1081,7 +1107,7 @@ static int gemm_check_w(const void *w, int64_t n, int64_t granule, int64_t k) {
 using namespace cascade;
 
 // Split K.  Where 256-row tiles would keep at most half of the CUs busy
-// (prompts of 17 to about 1000 rows over N = 4096: down_proj), K is
+// (prompts of 17 to 1280 rows over N = 4096: down_proj), K is
 // split over up to kSplitMax rows of workgroups, each writing
 // an fp32 partial tile into the caller's workspace; a second launch sums
 // the partials in split order and applies the element-wise epilogue at the
@@ -1089,7 +1115,11 @@ using namespace cascade;
 // add).  The partials associate the K sum differently from one pass, so a
 // result may differ from the one-pass tile in the last bf16 place, within
 // the same rounding bound.  Up to 256 rows the streaming kernel writes the
-// partials (stream_split_plan), past that the 256-row tiles.  Over a short K
+// partials (stream_split_plan), past that 256 x 128 tiles, or 160 x 256
+// tiles where, at kLowRound a tile, their more numerous splits are shorter
+// (down_proj: 320 rows 53.7 -> 50.1 us, 613 rows 86.6 -> 73.4, 768 rows
+// 104 -> 92; 1100 and 1280 rows, whose 160 tiles of 256 x 128 do not split,
+// 192 -> 120 and 218 -> 127).  Over a short K
 // (K < 8192: o_proj) up to 128 rows the one-pass streaming kernel ends
 // before a split launch and its reduction (M = 64: 13.8 against 15.2 us),
 // so the workspace those shapes ask for is checked and left alone.
@@ -1101,21 +1131,27 @@ struct SplitPlan {
   int splits;  // 1: no split
   int per;     // slabs per split
   StreamPlan stream;  // fm: the streaming kernel writes the partials
+  bool low;           // 160 x 256 tiles write them
 };
 
-static SplitPlan split_plan(int64_t m, int64_t n, int64_t k, int cus) {
-  SplitPlan p{1, 0, {0, 0, 1}};
+static SplitPlan split_plan(int64_t m, int64_t n, int64_t k, int cus, bool low_tiles = true) {
+  SplitPlan p{1, 0, {0, 0, 1}, false};
   // 16 rows and fewer: one pass streams the weight faster (M = 6,
   // down_proj: 23.3 us one pass, 21 + 4.7 split)
   if (m <= 16 || n % 8 != 0 || k % kTileK != 0) return p;
   // short K past 128 rows: one pass finishes first
   // (o_proj, M = 192..1024: 22.0..33.8 us one pass, 23.3..42.8 split)
   if (k < 8192 && m > kShortPrompt) return p;
-  const int64_t tiles = (m + 255) / 256 * ((n + kTileN - 1) / kTileN);
-  if (2 * tiles > cus) return p;
   const int64_t slabs = k / kTileK;
-  int64_t sp = std::min<int64_t>(std::min<int64_t>(kSplitMax, cus / tiles),
-                                 slabs / kSplitMinSlabs);
+  auto runs = [&](int64_t tiles) {
+    return std::min<int64_t>(std::min<int64_t>(kSplitMax, cus / tiles), slabs / kSplitMinSlabs);
+  };
+  int64_t sp = runs((m + 255) / 256 * ((n + kTileN - 1) / kTileN));
+  if (low_tiles && m > 256) {
+    const int64_t low = runs((m + 159) / 160 * ((n + 255) / 256));
+    p.low = low >= 2 && kLowRound * std::max<int64_t>(sp, 1) < low;
+    if (p.low) sp = low;
+  }
   if (sp < 2) return p;
   p.stream = stream_split_plan(m, n, k, cus);
   if (p.stream.fm) sp = p.stream.splits;
@@ -1168,10 +1204,13 @@ static int gemm_split_k(const GemmArgs &a, const SplitPlan &p, void *ws,
   b.ldy = a.n0;
   b.split_slabs = p.per;
   b.split_stride = part;
-  hipError_t e = p.stream.fm
-                     ? launch_stream(kGemmF32, p.stream, b, s)
-                     : launch_tiles<kGemmF32, kTileK, GemmTile256, 3>(
-                           b, (a.n0 + kTileN - 1) / kTileN, gemm_device_cus(s), s, p.splits);
+  const int cus = gemm_device_cus(s);
+  hipError_t e =
+      p.stream.fm ? launch_stream(kGemmF32, p.stream, b, s)
+      : p.low     ? launch_tiles<kGemmF32, kTileK, GemmTile160, 3>(b, (a.n0 + 255) / 256, cus, s,
+                                                                   p.splits)
+                  : launch_tiles<kGemmF32, kTileK, GemmTile256, 3>(
+                        b, (a.n0 + kTileN - 1) / kTileN, cus, s, p.splits);
   if (e != hipSuccess) return e;
   GemmArgs r = a;
   r.yf = static_cast<float *>(ws);
@@ -1235,7 +1274,14 @@ static int gemm_ws(int epi, const void *x, const void *w, const void *aux,
                    void *y, int64_t m, int64_t n, int64_t k, void *workspace,
                    size_t workspace_bytes, void *stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const SplitPlan p = split_plan(m, n, k, gemm_device_cus(s));
+  SplitPlan p = split_plan(m, n, k, gemm_device_cus(s));
+  // where only the 160-row tiles split, a call without their workspace runs
+  // the one pass
+  if (p.low && (workspace == nullptr ||
+                workspace_bytes < static_cast<size_t>(p.splits) * m * n * sizeof(float))) {
+    const SplitPlan one = split_plan(m, n, k, gemm_device_cus(s), false);
+    if (one.splits == 1) p = one;
+  }
   if (p.splits == 1)
     return gemm_plain(epi, x, w, aux, y, m, n, k, stream);
   if (int e = gemm_check_x(x, m, k)) return e;
