@@ -247,19 +247,29 @@ class VocabStreamingRuntime:
                 raise RuntimeError("a full_pinned store must hold the LM head "
                                    "in page-locked memory")
             return rows
-        self._prestage(chunk)  # no-op when already queued
+        if chunk not in self._prestaged:
+            # chunks are copied in order, so another one in the half is left
+            # over from a call that never reached its LM head (a run that
+            # raised, or one that nobody finished)
+            for other in [c for c in self._prestaged if c % 2 == chunk % 2]:
+                self._drop_prestaged(other)
+            self._prestage(chunk)
         return self._prestaged.pop(chunk).result()
+
+    def _drop_prestaged(self, chunk):
+        """Forget a staged chunk once its staging job is off the half."""
+
+        try:
+            self._prestaged.pop(chunk).result()
+        except Exception:  # the call that queued it never used it
+            pass
 
     def quiesce(self):
         """Wait for the staging jobs still reading the store's arena (called
         by the store before its bytes change)."""
 
-        for future in list(self._prestaged.values()):
-            try:
-                future.result()
-            except Exception:  # the call that queued it already raised
-                pass
-        self._prestaged = {}
+        for chunk in list(self._prestaged):
+            self._drop_prestaged(chunk)
         self._deferred = set()
 
     def _copy_chunk(self, chunk):

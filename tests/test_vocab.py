@@ -249,3 +249,62 @@ def test_staged_halves_are_copied_before_they_are_filled_again(chunks):
         assert copied[first:] == list(range(chunks))
     # the next call's first chunks are staged behind the last copies
     assert [h for h in holds if h is not None] == list(range(min(2, chunks)))
+
+
+@pytest.mark.parametrize("chunks", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("abandoned", [0, 1, 2])
+def test_staged_chunks_of_a_call_without_an_lm_head_are_dropped(chunks, abandoned):
+    # A run copies the first chunks and has the two after them staged; one
+    # that raises or is never finished leaves those in the pinned halves.
+    # The next call copies its own chunks in order, from halves nothing else
+    # is being staged into.
+    from types import SimpleNamespace
+
+    from layer_streaming.vocab import VocabStreamingRuntime
+
+    vocab = VocabStreamingRuntime.__new__(VocabStreamingRuntime)
+    holds, running, copied = [None, None], [None, None], []
+
+    class Staging:
+        def __init__(self, half, chunk):
+            self.half, self.chunk = half, chunk
+
+        def result(self):
+            if running[self.half] is self:
+                running[self.half] = None
+            return self.chunk
+
+    def stage_into(target, source, waits):
+        half, chunk = target[0].item(), int(source[0])
+        assert running[half] is None  # no job still writes the half
+        assert all(c % 2 != half for c in vocab._prestaged)  # nor is it in use
+        last = [c for c in copied if c % 2 == half][-1:]
+        assert list(waits) == ["ready {}".format(c) for c in last]
+        holds[half], running[half] = chunk, Staging(half, chunk)
+        return running[half]
+
+    def slot_copy(slot, kind, chunk, source, nbytes, ready, pair):
+        assert source == chunk == holds[slot] and running[slot] is None
+        copied.append(chunk)
+
+    vocab.vocab = SimpleNamespace(chunk_count=chunks, hidden_size=1,
+                                  chunk_bounds=lambda c: (c, c + 1),
+                                  lm_head_key="head")
+    vocab.store = SimpleNamespace(
+        tensor=lambda key: torch.arange(chunks).view(-1, 1), stage_into=stage_into)
+    vocab.transformer_runtime = SimpleNamespace(
+        slot_copy=slot_copy, stage_call_ahead=vocab._prestage_first_chunks)
+    vocab.head_staging_slots = [torch.tensor([0]), torch.tensor([1])]
+    vocab.profile, vocab._staged = False, True
+    vocab._ready = ["ready {}".format(c) for c in range(chunks)]
+    vocab._staging_read, vocab._prestaged, vocab._deferred = [None, None], {}, set()
+    for _ in range(2):
+        for _ in range(2):  # two calls in a row end behind these copies
+            vocab._prestage_first_chunks()
+            for slot in range(abandoned):
+                vocab._copy_first_chunk(slot)
+        vocab._prestage_first_chunks()
+        first = len(copied)
+        for chunk in range(chunks):
+            vocab._copy_chunk(chunk)
+        assert copied[first:] == list(range(chunks))
