@@ -1273,6 +1273,8 @@ extern "C" int cascade_gemm_residual_bf16(const void *x, const void *w,
 static int gemm_ws(int epi, const void *x, const void *w, const void *aux,
                    void *y, int64_t m, int64_t n, int64_t k, void *workspace,
                    size_t workspace_bytes, void *stream) {
+  if (int e = gemm_check_x(x, m, k)) return e;
+  if (int e = gemm_check_w(w, n, 1, k)) return e;
   hipStream_t s = static_cast<hipStream_t>(stream);
   SplitPlan p = split_plan(m, n, k, gemm_device_cus(s));
   // where only the 160-row tiles split, a call without their workspace runs
@@ -1284,8 +1286,6 @@ static int gemm_ws(int epi, const void *x, const void *w, const void *aux,
   }
   if (p.splits == 1)
     return gemm_plain(epi, x, w, aux, y, m, n, k, stream);
-  if (int e = gemm_check_x(x, m, k)) return e;
-  if (int e = gemm_check_w(w, n, 1, k)) return e;
   if (y == nullptr || workspace == nullptr || (epi == kGemmResidual && aux == nullptr))
     return CASCADE_EINVAL;
   if (!aligned16(y) || !aligned16(workspace) || (aux != nullptr && !aligned16(aux)))

@@ -78,6 +78,11 @@ def test_argument_checks_reject_without_launching():
                                              20, need, None) == 1002
     assert lib.cascade_gemm_ws_bf16(16, 16, 16, 64, 4096, 14336, 16, need - 4,
                                     None) == 1004
+    # no columns: refused before the split is planned
+    for m, n, k in ((17, 0, 14336), (300, 0, 14336), (64, -8, 14336), (64, 0, 4096)):
+        assert lib.cascade_gemm_ws_bf16(16, 16, 16, m, n, k, 16, need, None) == 1001
+        assert lib.cascade_gemm_residual_ws_bf16(16, 16, 16, 16, m, n, k, 16, need,
+                                                 None) == 1001
     # prefill attention: cache positions past + tokens are limited to 2^24,
     # head_dim to 128 and n_q_heads to 4 n_kv_heads
     pos = 1 << 24
