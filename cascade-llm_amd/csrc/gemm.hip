@@ -1277,9 +1277,10 @@ static int gemm_ws(int epi, const void *x, const void *w, const void *aux,
   if (int e = gemm_check_w(w, n, 1, k)) return e;
   hipStream_t s = static_cast<hipStream_t>(stream);
   SplitPlan p = split_plan(m, n, k, gemm_device_cus(s));
-  // where only the 160-row tiles split, a call without their workspace runs
-  // the one pass
-  if (p.low && (workspace == nullptr ||
+  // where only the 160-row tiles split, a call without their workspace, or
+  // whose workspace or residual is not 16-byte aligned, runs the one pass
+  if (p.low && (workspace == nullptr || !aligned16(workspace) ||
+                (aux != nullptr && !aligned16(aux)) ||
                 workspace_bytes < static_cast<size_t>(p.splits) * m * n * sizeof(float))) {
     const SplitPlan one = split_plan(m, n, k, gemm_device_cus(s), false);
     if (one.splits == 1) p = one;

@@ -99,3 +99,19 @@ def test_low_split(gpu_device, m, n, k, splits, refused):
         _hip.gemm(xd, wd, y, workspace=ws[:16])
         _hip.gemm(xd, wd, out)
         assert torch.equal(out, y)
+
+
+def test_low_split_takes_what_the_one_pass_takes(gpu_device):
+    # where only these tiles split, an unaligned workspace is left alone and
+    # an unaligned residual is read element by element, as by the one pass
+    dev, (m, n, k) = gpu_device, (1100, 4096, 8192)
+    x, w = cases.normal_bf16((m, k), 731).to(dev), cases.normal_bf16((n, k), 732, 0.02).to(dev)
+    need = _hip.gemm_workspace_bytes(m, n, k)
+    ws = torch.empty(need + 16, dtype=torch.uint8, device=dev)
+    shifted = cases.normal_bf16((m * n + 1,), 733).to(dev)[1:].view(m, n)
+    one, y, out = (torch.empty((m, n), dtype=BF16, device=dev) for _ in range(3))
+    _hip.gemm(x, w, one)
+    _hip.gemm(x, w, y, workspace=ws[4:])
+    assert torch.equal(y, one)
+    _hip.gemm_residual(x, w, shifted, out, workspace=ws)
+    assert torch.equal(out, shifted + one)
