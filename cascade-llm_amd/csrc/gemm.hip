@@ -1106,9 +1106,9 @@ static int gemm_check_w(const void *w, int64_t n, int64_t granule, int64_t k) {
 
 using namespace cascade;
 
-// Split K.  Where 256-row tiles would keep at most half of the CUs busy
-// (prompts of 17 to 1280 rows over N = 4096: down_proj), K is
-// split over up to kSplitMax rows of workgroups, each writing
+// Split K.  Where 256-row tiles would keep at most half of the CUs busy over
+// a long K (K >= 8192; prompts of 17 to 1280 rows over N = 4096: down_proj),
+// K is split over up to kSplitMax rows of workgroups, each writing
 // an fp32 partial tile into the caller's workspace; a second launch sums
 // the partials in split order and applies the element-wise epilogue at the
 // same rounding points as the one-pass tile (bf16(sum), then the residual
@@ -1119,13 +1119,12 @@ using namespace cascade;
 // tiles where, at kLowRound a tile, their more numerous splits are shorter
 // (down_proj: 320 rows 53.7 -> 50.1 us, 613 rows 86.6 -> 73.4, 768 rows
 // 104 -> 92; 1100 and 1280 rows, whose 160 tiles of 256 x 128 do not split,
-// 192 -> 120 and 218 -> 127).  Over a short K
-// (K < 8192: o_proj) up to 128 rows the one-pass streaming kernel ends
-// before a split launch and its reduction (M = 64: 13.8 against 15.2 us),
-// so the workspace those shapes ask for is checked and left alone.
+// 192 -> 120 and 218 -> 127).  Over a short K (o_proj) one pass ends before
+// a split launch and its reduction (M = 64: 13.8 against 15.2 us;
+// M = 192 .. 1024: 22.0 .. 33.8 against 23.3 .. 42.8).
 constexpr int kSplitMax = 8;
 constexpr int kSplitMinSlabs = 8;  // 64-deep slabs per split, at least
-constexpr int kShortPrompt = 128;
+constexpr int64_t kSplitMinK = 8192;
 
 struct SplitPlan {
   int splits;  // 1: no split
@@ -1138,10 +1137,7 @@ static SplitPlan split_plan(int64_t m, int64_t n, int64_t k, int cus, bool low_t
   SplitPlan p{1, 0, {0, 0, 1}, false};
   // 16 rows and fewer: one pass streams the weight faster (M = 6,
   // down_proj: 23.3 us one pass, 21 + 4.7 split)
-  if (m <= 16 || n % 8 != 0 || k % kTileK != 0) return p;
-  // short K past 128 rows: one pass finishes first
-  // (o_proj, M = 192..1024: 22.0..33.8 us one pass, 23.3..42.8 split)
-  if (k < 8192 && m > kShortPrompt) return p;
+  if (m <= 16 || n % 8 != 0 || k % kTileK != 0 || k < kSplitMinK) return p;
   const int64_t slabs = k / kTileK;
   auto runs = [&](int64_t tiles) {
     return std::min<int64_t>(std::min<int64_t>(kSplitMax, cus / tiles), slabs / kSplitMinSlabs);
@@ -1300,11 +1296,6 @@ static int gemm_ws(int epi, const void *x, const void *w, const void *aux,
   a.y = static_cast<uint16_t *>(y);
   a.ldy = n;
   a.aux = static_cast<const uint16_t *>(aux);
-  if (k < 8192) {  // m <= kShortPrompt
-    if (workspace_bytes < static_cast<size_t>(p.splits) * m * n * sizeof(float))
-      return CASCADE_EWORKSPACE;
-    return gemm_plain(epi, x, w, aux, y, m, n, k, stream);
-  }
   return epi == kGemmResidual
              ? gemm_split_k<kGemmResidual>(a, p, workspace, workspace_bytes, s)
              : gemm_split_k<kGemmStore>(a, p, workspace, workspace_bytes, s);

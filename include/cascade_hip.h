@@ -240,10 +240,10 @@ int cascade_gemm_bf16(const void *x, const void *w, void *y, int64_t m,
 int cascade_gemm_residual_bf16(const void *x, const void *w,
                                const void *residual, void *y, int64_t m,
                                int64_t n, int64_t k, void *stream);
-/* The same two products with a workspace: where 256-row tiles would keep at
- * most half of the device's CUs busy (M > 16 rows, N a multiple of 8,
- * K a multiple of 64; 17..1024 prompt rows over N = 4096 with K = 14336,
- * down_proj, and 17..128 rows with K = 4096, o_proj), K is
+/* The same two products with a workspace: over a long K (K >= 8192, a
+ * multiple of 64; N a multiple of 8; M > 16 rows), where one pass's tiles
+ * would keep at most half of the device's CUs busy (17..1280 prompt rows over
+ * N = 4096 with K = 14336, down_proj), K is
  * split over up to 8 groups of workgroups writing fp32 partials into the
  * workspace, which a second launch sums in split order before the
  * epilogue (same rounding points; the sum's association may move a result
@@ -251,7 +251,11 @@ int cascade_gemm_residual_bf16(const void *x, const void *w,
  * one-pass GEMM and the workspace is not touched.  The workspace needs
  * cascade_gemm_workspace_bytes(m, n, k) bytes for the current device (0:
  * no split for this shape; a null workspace is then accepted), 16-byte
- * aligned; calls sharing one workspace must be ordered on one stream.
+ * aligned; so must the residual be where K splits.  A smaller or null
+ * workspace is refused, except where 256-row tiles would fill the device
+ * (1025..1280 rows over N = 4096): the call then runs the one-pass GEMM, and
+ * so it does there for a workspace or residual that is not aligned.  Calls
+ * sharing one workspace must be ordered on one stream.
  * Replace the same F.linear calls as the forms above.                     */
 size_t cascade_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int cascade_gemm_ws_bf16(const void *x, const void *w, void *y, int64_t m,

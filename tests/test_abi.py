@@ -78,6 +78,9 @@ def test_argument_checks_reject_without_launching():
                                              20, need, None) == 1002
     assert lib.cascade_gemm_ws_bf16(16, 16, 16, 64, 4096, 14336, 16, need - 4,
                                     None) == 1004
+    # a short K runs one pass at every row count and asks for no workspace
+    for m in (17, 64, 128, 1024):
+        assert lib.cascade_gemm_workspace_bytes(m, 4096, 4096) == 0
     # no columns: refused before the split is planned
     for m, n, k in ((17, 0, 14336), (300, 0, 14336), (64, -8, 14336), (64, 0, 4096)):
         assert lib.cascade_gemm_ws_bf16(16, 16, 16, m, n, k, 16, need, None) == 1001
