@@ -17,13 +17,17 @@
 // to LDS, up to 148 KB in flight; slab depth 64, 128 or 256 so that a step
 // moves 16 KB or more), nontemporal where one workgroup alone reads the
 // rows.  Waves 0-3 multiply the even 32-deep chunks of K, waves 4-7 the odd
-// ones, whatever the shape, so a product's sum does not depend on the tile
-// that computed it; the halves meet in LDS as an fp32 tile, from which the
+// ones, each into two sums in turn, so that no chain of fp32 additions is
+// longer than a quarter of K (error of a product against 64 bits, K = 4096:
+// 1.9e-7 of its norm, with one sum a wave 2.7e-7); a quarter holds the same
+// chunks whatever the shape of the workgroup.  The halves meet in LDS as an
+// fp32 tile, from which the
 // epilogue takes 4 columns (or 4 RoPE pairs) of a token at a time.
 // SwiGLU launches (and the logits of a whole vocabulary) start each tile at
 // another run of K: with every CU on the same columns of rows 8 KB apart
 // the same few channels serve all of them (112 rows a CU, loads alone:
-// 44.9 -> 36.2 us).  The runs differ between the tiles of one XCD (tile / 8):
+// 44.9 -> 36.2 us); the sums of those launches depend on the start, hence on
+// the tile, within the same bound.  The runs differ between the tiles of one XCD (tile / 8):
 // taken from the tile number itself they agree within an XCD (logits of
 // 26 rows: 259 us, 217 without any, 174 so).
 //
@@ -114,8 +118,10 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
   const int slabs = (count * 64 + S::BK - 1) / S::BK;
   constexpr bool kRotates = EPI == kGemmSwiglu || EPI == kGemmSilu || EPI == kGemmMul;
   // (in runs of 256 columns of K, whatever the slab depth: the products of
-  // a fused launch and of its halves then add in the same order)
-  const int rot = (kRotates || a.rotate) && a.k >= 256
+  // a fused launch and of its halves then add in the same order; a K of an
+  // odd number of 64-deep slabs would start the second round of them in the
+  // other sum)
+  const int rot = (kRotates || a.rotate) && a.k >= 256 && a.k % 128 == 0
                       ? tile / kXcds % static_cast<int>(a.k / 256) * (256 / S::BK)
                       : 0;
 
@@ -182,11 +188,13 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
   const int kg = wave / 4;
   const int wn = wave % S::WN;
   const int wm = (wave % 4) / S::WN;
-  f32x4 acc[S::FMW][S::FNW];
+  f32x4 acc[2][S::FMW][S::FNW];  // the half's chunks go to either sum in turn
 #pragma unroll
-  for (int i = 0; i < S::FMW; ++i)
+  for (int e = 0; e < 2; ++e)
 #pragma unroll
-    for (int j = 0; j < S::FNW; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < S::FMW; ++i)
+#pragma unroll
+      for (int j = 0; j < S::FNW; ++j) acc[e][i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   const int fl = S::CH == 8 ? (lr / 2) % 8 : lr;
   constexpr int KS = S::BK / 64;  // chunks of a wave's K half in a slab
   struct Frags {
@@ -207,18 +215,21 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
             b0 + (NR + 16 * min(wm + S::WM * i, FM - 1)) * S::RB + off);
     }
   };
-  auto multiply = [&](int slab, const Frags &f) __attribute__((always_inline)) {
+  // odd: an odd slab (64-deep slabs hold one chunk of the wave's half each)
+  auto multiply = [&](int slab, const Frags &f, auto odd) __attribute__((always_inline)) {
     int at = slab + rot;
     if (at >= slabs) at -= slabs;
     const int valid = count * 2 - at * (S::BK / 32);  // 32-deep chunks left
 #pragma unroll
     for (int q = 0; q < KS; ++q) {
       if (KS > 1 && 2 * q + kg >= valid) break;
+      constexpr int kOdd = decltype(odd)::value;
+      const int set = KS == 1 ? kOdd : q & 1;
 #pragma unroll
       for (int i = 0; i < S::FMW; ++i)
 #pragma unroll
         for (int j = 0; j < S::FNW; ++j)
-          acc[i][j] = mfma_16x16x32_bf16(f.w[q][j], f.x[q][i], acc[i][j]);
+          acc[set][i][j] = mfma_16x16x32_bf16(f.w[q][j], f.x[q][i], acc[set][i][j]);
     }
   };
   // Slab s in ring buffer s % STAGES.  Step s waits for this wave's loads of
@@ -242,23 +253,30 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
   publish(std::integral_constant<int, S::STAGES - 1>{});
   read_frags(0, f0);
   int buf = 0;
-  auto step = [&](int slab, const Frags &here, Frags &next) __attribute__((always_inline)) {
+  auto step = [&](int slab, const Frags &here, Frags &next, auto odd)
+      __attribute__((always_inline)) {
     publish(std::integral_constant<int, S::STAGES - 2>{});
     load_slab(slab + S::STAGES, buf);
     buf = buf + 1 == S::STAGES ? 0 : buf + 1;
     read_frags(buf, next);
-    multiply(slab, here);
+    multiply(slab, here, odd);
   };
+  constexpr std::integral_constant<int, 0> kEven;
+  constexpr std::integral_constant<int, 1> kOdd;
   int slab = 0;
   for (; slab + 2 <= slabs; slab += 2) {
-    step(slab, f0, f1);
-    step(slab + 1, f1, f0);
+    step(slab, f0, f1, kEven);
+    step(slab + 1, f1, f0, kOdd);
   }
-  if (slab < slabs) step(slab, f0, f1);
+  if (slab < slabs) step(slab, f0, f1, kEven);
   // every load landed and every LDS read done before the ring holds the tile
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
   __syncthreads();
+#pragma unroll
+  for (int i = 0; i < S::FMW; ++i)
+#pragma unroll
+    for (int j = 0; j < S::FNW; ++j) acc[0][i][j] += acc[1][i][j];
   float *tile_f = reinterpret_cast<float *>(ring);
   auto each = [&](auto f) {
 #pragma unroll
@@ -268,7 +286,7 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
         const int fi = wm + S::WM * i, fj = wn + S::WN * j;
         if (fi < FM && fj < S::FN)
           f(reinterpret_cast<f32x4 *>(tile_f + (16 * fi + lr) * S::PITCH + 16 * fj + 4 * g4),
-            acc[i][j]);
+            acc[0][i][j]);
       }
   };
   if (kg == 1) each([](f32x4 *p, const f32x4 &v) { *p = v; });

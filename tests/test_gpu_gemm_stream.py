@@ -91,3 +91,54 @@ def test_stream_qkv_split_equals_fused(gpu_device, m):
     v = ref.linear(x.cpu(), w[2].cpu()).view(m, 8, 128).transpose(0, 1)
     assert cases.compare(outs[0][2][:, 1:m + 1].cpu(), v)["ok"]
     assert int(outs[0][2][:, 0].abs().sum()) == 0
+
+
+@pytest.mark.parametrize("m,n", [(6, 8192), (64, 8192), (128, 8192), (6, 66048)])
+def test_stream_sums_are_quarters_of_k(gpu_device, m, n):
+    # rounding errors of a chain of fp32 additions grow as the root of its
+    # length: four chains leave half the error of one (tiles of more rows),
+    # two would leave 0.71 of it
+    dev, k = gpu_device, 4096
+    x = cases.normal_bf16((192, k), 331).to(dev)
+    w = cases.normal_bf16((n, k), 332, 0.02).to(dev)
+    exact = x[:m].double() @ w.double().t()
+    errors = []
+    for rows in (m, 192):
+        y = torch.empty((rows, n), dtype=torch.float32, device=dev)
+        _hip.gemm_f32out(x[:rows], w, y)
+        errors.append(float((y[:m].double() - exact).norm()))
+    assert errors[0] <= 0.6 * errors[1], errors
+
+
+@pytest.mark.parametrize("m,n,k", [(2, 65544, 256), (33, 65700, 640), (64, 128256, 896),
+                                   (128, 70000, 1024), (17, 66048, 576)])
+def test_stream_rotated_logits(gpu_device, m, n, k):
+    # more than 65536 columns: each tile starts at another 256 columns of K
+    # (640, 896: the last slab of 256 or 128 is short; 576: an odd number of
+    # 64-deep slabs, not rotated).  Bound of fp32 accumulation as above.
+    print("rotated logits m={} n={} k={}".format(m, n, k), flush=True)
+    dev = gpu_device
+    x = cases.normal_bf16((m, k), 341).to(dev)
+    w = cases.normal_bf16((n, k), 342, 0.05).to(dev)
+    y = torch.full((m, n), float("nan"), dtype=torch.float32, device=dev)
+    _hip.gemm_f32out(x, w, y)
+    exact = x.double() @ w.double().t()
+    bound = 2.0 ** -22 * (x.double().abs() @ w.double().abs().t())
+    assert bool(((y.double() - exact).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(16, 1024, 640), (33, 2048, 896), (100, 14336, 640),
+                                   (160, 14336, 768), (49, 4096, 1152)])
+def test_stream_rotated_swiglu_equals_its_halves(gpu_device, m, n, k):
+    # the fused launch and its halves walk K in slabs of other depths from the
+    # same starts, and add in the same order
+    dev = gpu_device
+    x = cases.normal_bf16((m, k), 351).to(dev)
+    wg, wu = (cases.normal_bf16((n, k), s, 0.05).to(dev) for s in (352, 353))
+    fused, gate, split = (torch.empty((m, n), dtype=BF16, device=dev) for _ in range(3))
+    _hip.gate_up_swiglu_gemm(x, wg, wu, fused)
+    _hip.gate_silu_gemm(x, wg, gate)
+    _hip.up_mul_gemm(x, wu, gate, split)
+    assert torch.equal(fused, split)
+    exact = F.silu(x.double() @ wg.double().t())
+    assert cases.compare(gate, exact.to(BF16).cpu())["ok"]
