@@ -14,9 +14,13 @@
 // tokens and twice or four times the weight rows each (stream_plan).
 //
 // K is walked in slabs through a ring of LDS buffers (buffer loads straight
-// to LDS, up to 148 KB in flight; slab depth 64, 128 or 256 so that a step
+// to LDS, up to 148 KB in flight; slab depth 64 to 512 so that a step
 // moves 16 KB or more), nontemporal where one workgroup alone reads the
-// rows.  Waves 0-3 multiply the even 32-deep chunks of K, waves 4-7 the odd
+// rows.  Up to 16 rows over few columns a launch is a chain of steps with
+// little to load in each: 512-deep slabs halve them, and waves that would
+// repeat another one's fragment leave the LDS alone (M = 6, N = 1024: 8.0 ->
+// 6.8 us, N = 4096 10.0 -> 9.5; without the nontemporal hint 0.5 to 1.0 us
+// less over K = 2048, 2.9 more over K = 14336).  Waves 0-3 multiply the even 32-deep chunks of K, waves 4-7 the odd
 // ones, each into two sums in turn, so that no chain of fp32 additions is
 // longer than a quarter of K (error of a product against 64 bits, K = 4096:
 // 1.9e-7 of its norm, with one sum a wave 2.7e-7); a quarter holds the same
@@ -60,7 +64,7 @@ struct StreamShape {
   static constexpr int MT = 16 * FM;          // token rows of a workgroup
   static constexpr int FN = (NR + 15) / 16;   // fragments of its weight rows
   static constexpr int ROWS = NR + MT;
-  static constexpr int BK = ROWS >= 128 ? 64 : ROWS >= 64 ? 128 : 256;
+  static constexpr int BK = ROWS >= 128 ? 64 : ROWS >= 64 ? 128 : ROWS > 32 ? 256 : 512;
   static constexpr int RB = 2 * BK;           // bytes of one row in a slab
   static constexpr int CH = BK / 8;           // 16-byte chunks of it
   static constexpr int RPI = 1024 / RB;       // rows per load instruction
@@ -73,7 +77,7 @@ struct StreamShape {
   // starts or stores (M = 26: 174 -> 168 us, M = 64: 194 -> 187)
   static constexpr bool TWO = NR == 128 && 2 * 3 * SLAB <= 158000;
   static constexpr int FIT = (TWO ? 79000 : 151552) / SLAB;
-  static constexpr int STAGES = FIT > 12 ? 12 : FIT;
+  static constexpr int STAGES = BK == 512 ? 3 : FIT > 12 ? 12 : FIT;
   static constexpr int PITCH = 16 * FN + 4;   // floats per token of the staged tile
   static constexpr int LDS = std::max(STAGES * SLAB, MT * PITCH * 4);
   // 4 waves of each K half share the fragments
@@ -121,8 +125,8 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
   // a fused launch and of its halves then add in the same order; a K of an
   // odd number of 64-deep slabs would start the second round of them in the
   // other sum)
-  const int rot = (kRotates || a.rotate) && a.k >= 256 && a.k % 128 == 0
-                      ? tile / kXcds % static_cast<int>(a.k / 256) * (256 / S::BK)
+  const int rot = S::BK <= 256 && (kRotates || a.rotate) && a.k >= 256 && a.k % 128 == 0
+                      ? tile / kXcds % static_cast<int>(a.k / 256) * (256 / std::min(256, S::BK))
                       : 0;
 
   // load instruction t of this wave: wave + 8 t of the slab's NI (weight
@@ -165,7 +169,7 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
     const int f = S::CH == 8 ? (sr / 2) % 8 : sr % 16;
     voff[t] = static_cast<int>(row * k_bytes) + 128 * piece0 + 16 * ((lane % S::CH) ^ f);
   }
-  const bool stream_w = gridDim.y == 1;
+  const bool stream_w = gridDim.y == 1 && (S::BK < 512 || a.k >= 4096);
   const uint32_t ring_lds = lds_address(ring);
   auto load_slab = [&](int slab, int buf) {
     int at = min(slab, slabs - 1) + rot;
@@ -188,6 +192,8 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
   const int kg = wave / 4;
   const int wn = wave % S::WN;
   const int wm = (wave % 4) / S::WN;
+  // waves left without a fragment of their own only load
+  const bool idle = S::WM >= 2 * FM && wm >= FM;
   f32x4 acc[2][S::FMW][S::FNW];  // the half's chunks go to either sum in turn
 #pragma unroll
   for (int e = 0; e < 2; ++e)
@@ -201,6 +207,7 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
     u32x4 w[KS][S::FNW], x[KS][S::FMW];
   };
   auto read_frags = [&](int buf, Frags &f) __attribute__((always_inline)) {
+    if (idle) return;
     const unsigned char *b0 = ring + buf * S::SLAB + lr * S::RB;
 #pragma unroll
     for (int q = 0; q < KS; ++q) {
@@ -220,6 +227,7 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
     int at = slab + rot;
     if (at >= slabs) at -= slabs;
     const int valid = count * 2 - at * (S::BK / 32);  // 32-deep chunks left
+    if (idle) return;
 #pragma unroll
     for (int q = 0; q < KS; ++q) {
       if (KS > 1 && 2 * q + kg >= valid) break;

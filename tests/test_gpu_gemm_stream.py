@@ -142,3 +142,27 @@ def test_stream_rotated_swiglu_equals_its_halves(gpu_device, m, n, k):
     assert torch.equal(fused, split)
     exact = F.silu(x.double() @ wg.double().t())
     assert cases.compare(gate, exact.to(BF16).cpu())["ok"]
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 40, 512), (16, 1000, 576), (7, 520, 1088), (9, 4096, 1984),
+                                   (16, 2056, 4160), (3, 8, 64)])
+def test_stream_deep_slabs(gpu_device, m, n, k):
+    # up to 16 rows and 16 columns a workgroup: 512-deep slabs, K below, at and
+    # past whole ones, with and without the nontemporal hint (K >= 4096)
+    print("deep slabs m={} n={} k={}".format(m, n, k), flush=True)
+    dev = gpu_device
+    x, w = cases.normal_bf16((m, k), 361), cases.normal_bf16((n, k), 362, 0.05)
+    res = cases.normal_bf16((m, n), 363).to(dev)
+    xd, wd = x.to(dev), w.to(dev)
+    y, out, gate, prod = (torch.empty((m, n), dtype=BF16, device=dev) for _ in range(4))
+    _hip.gemm(xd, wd, y)
+    assert linear_bound_report(y, x, w) <= 1.0
+    _hip.gemm_residual(xd, wd, res, out)
+    assert torch.equal(out, res + y)
+    yf = torch.empty((m, n), dtype=torch.float32, device=dev)
+    _hip.gemm_f32out(xd, wd, yf)
+    assert torch.equal(yf.to(BF16), y)
+    _hip.gate_silu_gemm(xd, wd, gate)
+    assert cases.compare(gate.cpu(), F.silu(y.cpu()))["ok"]
+    _hip.up_mul_gemm(xd, wd, gate, prod)
+    assert torch.equal(prod, gate * y)
