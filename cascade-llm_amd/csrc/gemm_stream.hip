@@ -6,11 +6,15 @@
 // then by what each CU takes in besides, since a CU's loads return in order
 // and the X lines that hit its XCD's L2 queue with the weight lines that do
 // not.  So one workgroup per CU owns a run of weight rows that divides the
-// matrix evenly over the CUs (112 of the 28672 gate and up rows, 24 of the
-// 6144 q|k|v rows, 16 of o_proj's 4096; not a power of two, so no round of
-// tiles is part empty) and walks all of K once: the ramp of a launch is paid
+// matrix over the CUs (112 of the 28672 gate and up rows, 24 of the
+// 6144 q|k|v rows, 16 of o_proj's 4096: not a power of two, so these rounds
+// are full; other widths take the next built count, which leaves at most
+// half of the CUs idle: gate|up of 4096, M = 6: 15.1 us on 32 rows, 23.2 on
+// 112; logits of 8192 17.6 on 32, 24.3 on 128) and walks all of K once: the
+// ramp of a launch is paid
 // once, and every token row is read once per workgroup.  Where the token
-// rows would outweigh the weight rows, 2 or 4 workgroups take a share of the
+// rows would outweigh the weight rows, 2 or 4 workgroups on one XCD take a
+// share of the
 // tokens and twice or four times the weight rows each (stream_plan).
 //
 // K is walked in slabs through a ring of LDS buffers (buffer loads straight
@@ -113,6 +117,7 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
   const int lr = lane & 15;
   const int g4 = lane >> 4;
   const int tile = static_cast<int>(blockIdx.x);
+  if (tile >= a.tiles) return;  // padding: the whole workgroup
   const int64_t row0 = static_cast<int64_t>(blockIdx.y) * S::MT;
   const int64_t k_bytes = a.k * 2;
   // this split's 64-deep pieces of K
@@ -120,12 +125,16 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
   const int piece0 = a.split_slabs ? static_cast<int>(blockIdx.z) * a.split_slabs : 0;
   const int count = a.split_slabs ? min(a.split_slabs, pieces - piece0) : pieces;
   const int slabs = (count * 64 + S::BK - 1) / S::BK;
-  constexpr bool kRotates = EPI == kGemmSwiglu || EPI == kGemmSilu || EPI == kGemmMul;
+  // (not with 512-deep slabs, whose runs would be longer: one token fragment
+  // and up to 16 rows of each matrix)
+  constexpr bool kRotates = EPI == kGemmSwiglu ? FM > 1 || NR > 32
+                                               : (EPI == kGemmSilu || EPI == kGemmMul) &&
+                                                     (FM > 1 || NR > 16);
   // (in runs of 256 columns of K, whatever the slab depth: the products of
   // a fused launch and of its halves then add in the same order; a K of an
   // odd number of 64-deep slabs would start the second round of them in the
   // other sum)
-  const int rot = S::BK <= 256 && (kRotates || a.rotate) && a.k >= 256 && a.k % 128 == 0
+  const int rot = (kRotates || (S::BK <= 256 && a.rotate)) && a.k >= 256 && a.k % 128 == 0
                       ? tile / kXcds % static_cast<int>(a.k / 256) * (256 / std::min(256, S::BK))
                       : 0;
 
@@ -422,8 +431,12 @@ static hipError_t launch_stream_shape(const GemmArgs &args, int64_t n, hipStream
   const int64_t tiles = (n + NR - 1) / NR;
   const int64_t mt = (a.m + 16 * FM - 1) / (16 * FM);
   if (tiles > 0x7fffffff || mt > 65535) return static_cast<hipError_t>(CASCADE_ESHAPE);
+  a.tiles = static_cast<int32_t>(tiles);
+  // the workgroups that share a tile's weight rows must run on one XCD, or
+  // each reads them from memory again
+  const int64_t grid = mt > 1 ? (tiles + kXcds - 1) / kXcds * kXcds : tiles;
   return launch_kernel(gemm_stream_kernel<EPI, FM, NR>,
-                       dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(mt),
+                       dim3(static_cast<unsigned>(grid), static_cast<unsigned>(mt),
                             static_cast<unsigned>(splits)),
                        dim3(512), 0, s, a);
 }
@@ -455,9 +468,9 @@ using StreamFms = Ints<1, 2, 3, 4, 5, 6, 8, 10>;
 using StreamFmsQkv = Ints<1, 2, 3, 4, 5>;
 using StreamRows = Ints<16, 32, 64, 112>;              // plain, residual
 using StreamRowsQkv = Ints<16, 24, 32, 48, 64, 96>;
-using StreamRowsSwiglu = Ints<16, 112>;
-using StreamRowsHalf = Ints<8, 56>;                    // silu, mul: half of swiglu's
-using StreamRowsF32 = Ints<16, 64, 128>;               // logits; split-K partials
+using StreamRowsSwiglu = Ints<16, 32, 64, 112>;
+using StreamRowsHalf = Ints<8, 16, 32, 56>;                    // silu, mul: half of swiglu's
+using StreamRowsF32 = Ints<16, 32, 64, 112, 128>;      // logits; split-K partials
 
 template <int... V>
 static int at_least(Ints<V...>, int64_t want) {  // smallest built value >= want, or 0
@@ -482,7 +495,7 @@ static int rows_for(int epi, int64_t want) {
     case kGemmSwiglu: return pick(StreamRowsSwiglu{});
     case kGemmSilu:
     case kGemmMul: return pick(StreamRowsHalf{});
-    case kGemmF32: return want <= 16 ? 16 : 128;
+    case kGemmF32: return pick(StreamRowsF32{});
     default: return pick(StreamRows{});
   }
 }
@@ -490,25 +503,39 @@ static int rows_for(int epi, int64_t want) {
 // Up to 256 rows over at most 24 weight rows a CU (q|k|v, o, k, v), 160 over
 // more (gate|up at M = 157: 59.2 us against 73.6 on 128-row tiles), 128 for
 // logits (M = 128: 230 us against 250 on 256 x 256 tiles; M = 157: 266
-// against 250).  Shapes by M, each measured best at N = 4096 / 6144 over
-// K = 4096: one token tile up to 48 rows (M = 45: 13.0 us, two 14.5), two up
+// against 250).  Past 128 rows over 32 to 64 weight rows a CU one round of
+// tiles is shorter (M = 160: N = 10240 31.0 us, 35.0 here; 14336 36.6, 38.5;
+// 20480, two rounds, 62.8, 51.3), except for q|k|v, whose launches a matrix
+// at a time must add like the fused one.
+// Token tiles by M, each measured best at N = 4096 / 6144 over
+// K = 4096: one up to 48 rows (M = 45: 13.0 us, two 14.5), two up
 // to 112 (M = 100: 15.0, one 18.2; q|k|v to 160: 22.7, four 23.4), then four
-// (M = 157: 17.1, two 19.3).
+// (M = 157: 17.1, two 19.3); always one past 48 weight rows a CU, where the
+// weights outweigh the tokens again (M = 64: N = 14336 28.0 us, two 31.6;
+// N = 8192, M = 100: two 21.6, one 26.7).
 StreamPlan stream_plan(int epi, int64_t m, int64_t n, int cus) {
   const StreamPlan none{0, 0, 1};
-  const bool paired = epi == kGemmSwiglu || epi == kGemmSilu || epi == kGemmMul;
-  const int64_t narrow = 24 * static_cast<int64_t>(cus);
-  if (m > (epi == kGemmF32 ? 128 : paired || n > narrow ? 160 : 256)) return none;
+  const bool half = epi == kGemmSilu || epi == kGemmMul;
+  const bool paired = epi == kGemmSwiglu || half;
+  // weight rows of the launch, of a half those of both, so that the fused
+  // launch and its halves take the same tiles
+  const int64_t all = half ? 2 * n : n;
+  if (m > (epi == kGemmF32 ? 128 : paired || all > 24 * static_cast<int64_t>(cus) ? 160 : 256))
+    return none;
+  if (m > 128 && epi != kGemmQkvRope && all > 32 * static_cast<int64_t>(cus) &&
+      all <= 64 * static_cast<int64_t>(cus))
+    return none;
   // token tiles wanted: the bytes a workgroup loads are its weight rows plus
   // its tokens' rows, least where the two are about equal
   const int64_t per_cu = (n + cus - 1) / cus;
-  const int64_t want = paired || epi == kGemmF32 || m <= 48 ? 1
-                       : m <= (epi == kGemmQkvRope ? 160 : 112) ? 2 : 4;
+  const int64_t want = m <= 48 || all > 48 * static_cast<int64_t>(cus) ? 1
+                       : m <= (epi == kGemmQkvRope ? 160 : 112)        ? 2
+                                                                       : 4;
   StreamPlan p;
   p.rows = rows_for(epi, per_cu * want);
   const int64_t tiles = (n + p.rows - 1) / p.rows;
   const int64_t frags = (m + 15) / 16;
-  const int64_t mt = paired ? 1 : std::max<int64_t>(1, std::min(cus / tiles, frags));
+  const int64_t mt = std::max<int64_t>(1, std::min(cus / tiles, frags));
   const int64_t fm = (frags + mt - 1) / mt;
   p.fm = epi == kGemmQkvRope ? at_least(StreamFmsQkv{}, fm) : at_least(StreamFms{}, fm);
   p.splits = 1;

@@ -166,3 +166,33 @@ def test_stream_deep_slabs(gpu_device, m, n, k):
     assert cases.compare(gate.cpu(), F.silu(y.cpu()))["ok"]
     _hip.up_mul_gemm(xd, wd, gate, prod)
     assert torch.equal(prod, gate * y)
+
+
+@pytest.mark.parametrize("n", [3584, 4096, 5120, 7168])
+@pytest.mark.parametrize("m", [5, 16, 33, 100, 129, 160])
+def test_stream_widths(gpu_device, m, n):
+    # 32 and 64 gate and up rows a workgroup (16 and 32 in the halves), token
+    # tiles that share an XCD (tile counts that are no multiple of 8), 32 and
+    # 112 rows for logits; past 128 rows 5120 and 7168 gate rows run tiles
+    dev, k = gpu_device, 768
+    print("stream widths m={} n={}".format(m, n), flush=True)
+    x = cases.normal_bf16((m, k), 371).to(dev)
+    wg, wu = (cases.normal_bf16((n, k), s, 0.05).to(dev) for s in (372, 373))
+    fused, gate, split = (torch.empty((m, n), dtype=BF16, device=dev) for _ in range(3))
+    _hip.gate_up_swiglu_gemm(x, wg, wu, fused)
+    _hip.gate_silu_gemm(x, wg, gate)
+    _hip.up_mul_gemm(x, wu, gate, split)
+    assert torch.equal(fused, split)
+    product = x.double() @ wg.double().t()
+    assert cases.compare(gate.cpu(), F.silu(product).to(BF16).cpu())["ok"]
+    # all rows of both matrices in one product
+    both = torch.cat((wg, wu))
+    wide = torch.empty((m, 2 * n), dtype=torch.float32, device=dev)
+    y = torch.empty((m, 2 * n), dtype=BF16, device=dev)
+    _hip.gemm_f32out(x, both, wide)
+    _hip.gemm(x, both, y)
+    bound = 2.0 ** -22 * (x.double().abs() @ both.double().abs().t())
+    assert bool(((wide.double() - x.double() @ both.double().t()).abs() <= bound).all())
+    if m <= 128:
+        assert torch.equal(wide.to(BF16), y)
+    assert linear_bound_report(y, x.cpu(), both.cpu()) <= 1.0
