@@ -1115,7 +1115,7 @@ using namespace cascade;
 // add).  The partials associate the K sum differently from one pass, so a
 // result may differ from the one-pass tile in the last bf16 place, within
 // the same rounding bound.  Up to 256 rows the streaming kernel writes the
-// partials (stream_split_plan), past that 256 x 128 tiles, or 160 x 256
+// partials where it has enough runs (stream_split_plan), past that 256 x 128 tiles, or 160 x 256
 // tiles where, at kLowRound a tile, their more numerous splits are shorter
 // (down_proj: 320 rows 53.7 -> 50.1 us, 613 rows 86.6 -> 73.4, 768 rows
 // 104 -> 92; 1100 and 1280 rows, whose 160 tiles of 256 x 128 do not split,
@@ -1124,6 +1124,12 @@ using namespace cascade;
 // M = 192 .. 1024: 22.0 .. 33.8 against 23.3 .. 42.8).
 constexpr int kSplitMax = 8;
 constexpr int kSplitMinSlabs = 8;  // 64-deep slabs per split, at least
+// Of 160 x 256 tiles: their ramp and the reduction of twice the partials
+// outweigh shorter runs (N = 4096, 304 rows, 8 splits against 4 of 256 x 128
+// tiles: K = 8192 43.8 and 36.9 us, 10240 47.7 and 42.5, 14336 50.2 and 54.5);
+// nor does a split pay where one pass is a single round of 128-row tiles
+// (N = 6144, K = 8192: 600 rows 75.7 us, one pass 68.9; 700 rows 78 and 110).
+constexpr int kLowMinSlabs = 28;
 constexpr int64_t kSplitMinK = 8192;
 
 struct SplitPlan {
@@ -1145,7 +1151,9 @@ static SplitPlan split_plan(int64_t m, int64_t n, int64_t k, int cus, bool low_t
   int64_t sp = runs((m + 255) / 256 * ((n + kTileN - 1) / kTileN));
   if (low_tiles && m > 256) {
     const int64_t low = runs((m + 159) / 160 * ((n + 255) / 256));
-    p.low = low >= 2 && kLowRound * std::max<int64_t>(sp, 1) < low;
+    const bool two_rounds = (m + 127) / 128 * ((n + kTileN - 1) / kTileN) > cus;
+    p.low = low >= 2 && kLowRound * std::max<int64_t>(sp, 1) < low &&
+            slabs >= kLowMinSlabs * low && (sp >= 2 || two_rounds);
     if (p.low) sp = low;
   }
   if (sp < 2) return p;

@@ -546,7 +546,11 @@ StreamPlan stream_plan(int epi, int64_t m, int64_t n, int cus) {
 // read 28 KB of every token row for 16 weight rows (M = 45: 36.3 us); 64 weight
 // rows over a quarter of K read 7 KB (22.9 us and 4.7 for the reduction).
 // 128 rows over an eighth past 112 token rows (M = 100: 28.8 against 27.9 us,
-// but twice the partials; M = 157: 37.5 against 32.9).
+// but twice the partials; M = 157: 37.5 against 32.9).  Over more columns
+// fewer runs fit, and 256 x 128 tiles with twice as many end first: two runs
+// of 64 rows past 64 token rows (8192 columns over K = 28672, M = 112: 111 us
+// tiles, 120 here; M = 64: 100, 101), two or three past 160 (N = 5120, M = 200:
+// 48, 54; N = 8192: 129, 156; four, N = 4096: 47.0, 45.5).
 StreamPlan stream_split_plan(int64_t m, int64_t n, int64_t k, int cus) {
   StreamPlan p{0, 0, 1};
   if (m <= 16 || m > 256 || k < 8192) return p;
@@ -555,7 +559,7 @@ StreamPlan stream_split_plan(int64_t m, int64_t n, int64_t k, int cus) {
   const int64_t tiles = (n + p.rows - 1) / p.rows * mt;
   const int64_t slabs = k / 64;
   const int64_t sp = std::min<int64_t>(std::min<int64_t>(8, cus / tiles), slabs / 8);
-  if (sp < 2) return p;
+  if (sp < (m <= 64 ? 2 : m <= 160 ? 3 : 4)) return p;
   p.fm = at_least(StreamFms{}, ((m + 15) / 16 + mt - 1) / mt);
   p.splits = static_cast<int>(sp);
   return p;

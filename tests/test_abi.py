@@ -81,6 +81,12 @@ def test_argument_checks_reject_without_launching():
     # a short K runs one pass at every row count and asks for no workspace
     for m in (17, 64, 128, 1024):
         assert lib.cascade_gemm_workspace_bytes(m, 4096, 4096) == 0
+    # splits: 160-row tiles only over long runs of K and where one pass takes
+    # two rounds, the streaming kernel past 160 rows only with four runs
+    for m, n, k, splits in ((304, 4096, 8192, 4), (304, 4096, 14336, 8), (600, 6144, 8192, 0),
+                            (700, 6144, 8192, 2), (200, 8192, 28672, 4), (200, 4096, 14336, 4),
+                            (100, 8192, 28672, 4), (64, 8192, 28672, 2)):
+        assert lib.cascade_gemm_workspace_bytes(m, n, k) == splits * m * n * 4, (m, n, k)
     # no columns: refused before the split is planned
     for m, n, k in ((17, 0, 14336), (300, 0, 14336), (64, -8, 14336), (64, 0, 4096)):
         assert lib.cascade_gemm_ws_bf16(16, 16, 16, m, n, k, 16, need, None) == 1001

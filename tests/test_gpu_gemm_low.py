@@ -74,9 +74,10 @@ def test_low_qkv_equals_split(gpu_device, m):
 
 
 @pytest.mark.parametrize("m,n,k,splits,refused", [
-    (257, 4096, 8192, 8, True), (320, 4096, 8256, 8, True), (613, 4088, 8192, 4, True),
+    (257, 4096, 14336, 8, True), (320, 4096, 14400, 8, True), (613, 4088, 8192, 4, True),
     (641, 4096, 8192, 3, True), (1100, 4096, 8192, 2, False)])
 def test_low_split(gpu_device, m, n, k, splits, refused):
+    # 28 slabs of K a split at least, so eight of them need K >= 14336
     print("low split m={} n={} k={}".format(m, n, k), flush=True)
     dev = gpu_device
     x, w = cases.normal_bf16((m, k), 721), cases.normal_bf16((n, k), 722, 0.02)
