@@ -117,7 +117,6 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
   const int lr = lane & 15;
   const int g4 = lane >> 4;
   const int tile = static_cast<int>(blockIdx.x);
-  if (tile >= a.tiles) return;  // padding: the whole workgroup
   const int64_t row0 = static_cast<int64_t>(blockIdx.y) * S::MT;
   const int64_t k_bytes = a.k * 2;
   // this split's 64-deep pieces of K
@@ -431,10 +430,13 @@ static hipError_t launch_stream_shape(const GemmArgs &args, int64_t n, hipStream
   const int64_t tiles = (n + NR - 1) / NR;
   const int64_t mt = (a.m + 16 * FM - 1) / (16 * FM);
   if (tiles > 0x7fffffff || mt > 65535) return static_cast<hipError_t>(CASCADE_ESHAPE);
-  a.tiles = static_cast<int32_t>(tiles);
-  // the workgroups that share a tile's weight rows must run on one XCD, or
-  // each reads them from memory again
-  const int64_t grid = mt > 1 ? (tiles + kXcds - 1) / kXcds * kXcds : tiles;
+  // The workgroups that share a tile's weight rows run on one XCD, or each
+  // reads them from memory again: up to 7 workgroups more in each row of
+  // them, past every weight row (their loads read zeros, they store nothing),
+  // while all fit the CUs.  (A test of the tile in the kernel made every
+  // launch 0.2 us longer.)
+  int64_t grid = (tiles + kXcds - 1) / kXcds * kXcds;
+  if (mt == 1 || grid * mt * splits > gemm_device_cus(s)) grid = tiles;
   return launch_kernel(gemm_stream_kernel<EPI, FM, NR>,
                        dim3(static_cast<unsigned>(grid), static_cast<unsigned>(mt),
                             static_cast<unsigned>(splits)),
