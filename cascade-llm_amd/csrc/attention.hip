@@ -846,13 +846,18 @@ __attribute__((amdgpu_waves_per_eu(HW / 2))) void prefill_attention_kernel(
 // 8 tokens instead of 32, from the L2 of the XCD that serves the KV head, so
 // past kShortTokens the traffic outweighs the shorter chain.  Against the
 // kernel above, from position 0: 6 tokens 5.8 -> 4.5 us, 45 10.6 -> 4.9, 157
-// 14.2 -> 6.6, 300 17.4 -> 8.8, 613 23.7 -> 20.3, 800 26.3 -> 26.8; after 4000
-// cached positions: 64 tokens 167 -> 44, 600 161 -> 137.  8 waves a
+// 14.2 -> 6.6, 300 17.4 -> 8.8, 613 23.7 -> 20.3, 800 26.3 -> 26.8; after
+// cached positions the walks lengthen alike, and the line holds (704 tokens
+// after 1000: 58.2 -> 49.7, 4000: 157 -> 129, 32000: 1105 -> 867).  It lies
+// where the workgroups of 8 KV heads fill the CUs: 16 heads reach it at 352
+// tokens (after 2000 positions 85.5 -> 71.6; 400 tokens 86.3, here 92.1; 704
+// 94.5, 145), 32 at 176 (150 tokens 82.8 -> 70.9; 300 88.5, here 120).  8 waves a
 // workgroup, and the next block's loads ahead of this one's products (two
 // register sets), were 5-10% slower.
 constexpr int kShortWaves = 4;
 constexpr int kShortTile = 8;
 constexpr int64_t kShortTokens = 704;
+constexpr int64_t kShortWorkgroups = 704;
 constexpr int kShortPitch = kAttnD + 4;  // floats per column of a merged block
 
 __global__ __launch_bounds__(kShortWaves *kWave) void prefill_short_kernel(PrefillArgs a) {
@@ -1259,12 +1264,14 @@ extern "C" int cascade_prefill_attention_bf16(
   a.past = static_cast<int32_t>(past);
   a.tokens = static_cast<int32_t>(tokens);
   a.q_row = static_cast<int32_t>(n_q_heads * head_dim);
-  const int tile = tokens <= kShortTokens ? kShortTile : kPrefillUnit;
+  const bool few = tokens <= kShortTokens &&
+                   (tokens + kShortTile - 1) / kShortTile * n_kv_heads <= kShortWorkgroups;
+  const int tile = few ? kShortTile : kPrefillUnit;
   a.units = static_cast<int32_t>((tokens + tile - 1) / tile);
   a.kv_heads = static_cast<int32_t>(n_kv_heads);
   a.scale_log2 = scale * kLog2e;
   a.out = static_cast<uint16_t *>(out);
-  if (tokens <= kShortTokens)
+  if (few)
     return launch_kernel(prefill_short_kernel,
                          dim3(static_cast<unsigned>(a.units * n_kv_heads)),
                          dim3(kShortWaves * kWave), 0, static_cast<hipStream_t>(stream), a);

@@ -1,7 +1,7 @@
 """Causal attention of short prompts (one workgroup per 8 tokens and KV head)
 at the edges of its tiles and of its range: token counts around 8 and around
 the 704-token switch to the lockstep kernel, cached positions around a
-32-position block, few KV heads, rows past the end poisoned with NaN.
+32-position block, few KV heads, many (16 switch at 352 tokens, 32 at 176), rows past the end poisoned with NaN.
 
 P enters the products rounded to bf16 (relative 2^-9 each, averaging), the
 result is rounded once more: 1e-2 + 1e-2 |b| as in test_gpu_prefill.py."""
@@ -18,7 +18,8 @@ DIM = 128
 
 @pytest.mark.parametrize("past,tokens,kv", [
     (0, 1, 8), (0, 7, 8), (0, 8, 1), (0, 9, 8), (5, 33, 3), (31, 1, 8), (32, 64, 2),
-    (300, 17, 8), (1000, 40, 8), (0, 703, 2), (0, 704, 8), (0, 705, 2), (37, 704, 1)])
+    (300, 17, 8), (1000, 40, 8), (0, 703, 2), (0, 704, 8), (0, 705, 2), (37, 704, 1),
+    (0, 352, 16), (9, 353, 16), (40, 176, 32), (0, 177, 32)])
 def test_short_prompt_attention(gpu_device, past, tokens, kv):
     print("short attention past={} tokens={} kv={}".format(past, tokens, kv), flush=True)
     heads, total, cap = 4 * kv, past + tokens, past + tokens + 9
