@@ -176,8 +176,9 @@ __global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(TopkArgs a) {
 
 // ---- up to kPassTopK of them: passes of a block-wide maximum, one per key.
 // Both launches over 128256 logits: 4.5 us for 1 key, 6.8 for 4, 7.8 for 5,
-// 12.7 for 10, 73.9 for 64; the sorts 7.8 for 5, 8.4 for 10, 14.1 for 64.
-constexpr int kPassTopK = 4;
+// 8.6 for 6, 12.7 for 10, 73.9 for 64; the sorts 7.8 for 5 and 6, 8.4 for 10,
+// 14.1 for 64.  Over 10 to 100: passes 6.8 for 5 keys, 7.6 for 6, sorts 7.2.
+constexpr int kPassTopK = 5;
 constexpr int kPassThreads = 256;
 constexpr int kPassWaves = kPassThreads / kWave;
 constexpr int kPassMaxSlots = kTopkMaxSpan / kPassThreads;  // keys per thread, at most

@@ -1,5 +1,5 @@
 """Exact top-k at the edges of its two selections: passes of a maximum for up
-to 4 keys, sorted 64-key lists from 5; row counts around the 64-lane chunks,
+to 5 keys, sorted 64-key lists from 6; row counts around the 64-lane chunks,
 the 1024-logit spans and several spans; ties, signed zeros, NaN and -inf."""
 
 import pytest
@@ -19,7 +19,7 @@ def _expected(values, k):
     return sorted(range(len(values)), key=order)[:k]
 
 
-@pytest.mark.parametrize("top_k", [1, 4, 5, 33, 63, 64])
+@pytest.mark.parametrize("top_k", [1, 4, 5, 6, 33, 63, 64])
 @pytest.mark.parametrize("rows", [1, 63, 65, 1023, 1025, 4097, 20000])
 def test_topk_edges(gpu_device, rows, top_k):
     print("topk rows={} k={}".format(rows, top_k), flush=True)
