@@ -31,13 +31,18 @@
 // chunks whatever the shape of the workgroup.  The halves meet in LDS as an
 // fp32 tile, from which the
 // epilogue takes 4 columns (or 4 RoPE pairs) of a token at a time.
-// SwiGLU launches (and the logits of a whole vocabulary) start each tile at
-// another run of K: with every CU on the same columns of rows 8 KB apart
+// Wide SwiGLU launches and the logits of a whole vocabulary start each tile
+// at another run of K: with every CU on the same columns of rows 8 KB apart
 // the same few channels serve all of them (112 rows a CU, loads alone:
 // 44.9 -> 36.2 us); the sums of those launches depend on the start, hence on
-// the tile, within the same bound.  The runs differ between the tiles of one XCD (tile / 8):
-// taken from the tile number itself they agree within an XCD (logits of
-// 26 rows: 259 us, 217 without any, 174 so).
+// the tile, within the same bound.  The runs differ between the tiles of one
+// XCD (tile / 8): taken from the tile number itself they agree within an XCD
+// (logits of 26 rows: 259 us, 217 without any, 174 so).  It pays from about
+// 48 weight rows a CU on (gate|up of 7168, M = 33: 27.8 -> 23.1 us; of 4096
+// 16.4 -> 19.1).  The other kinds, and narrower logits, add in one order
+// whatever their width, so that a product does not depend on the columns
+// beside it, though it would shorten them too (14336 columns, M = 6: 24.8 ->
+// 20.6 us).
 //
 // Weights are the A operand, tokens the B operand: a lane then holds 4
 // consecutive weight rows, i.e. output columns, of one token.  8-row blocks
@@ -124,16 +129,11 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
   const int piece0 = a.split_slabs ? static_cast<int>(blockIdx.z) * a.split_slabs : 0;
   const int count = a.split_slabs ? min(a.split_slabs, pieces - piece0) : pieces;
   const int slabs = (count * 64 + S::BK - 1) / S::BK;
-  // (not with 512-deep slabs, whose runs would be longer: one token fragment
-  // and up to 16 rows of each matrix)
-  constexpr bool kRotates = EPI == kGemmSwiglu ? FM > 1 || NR > 32
-                                               : (EPI == kGemmSilu || EPI == kGemmMul) &&
-                                                     (FM > 1 || NR > 16);
   // (in runs of 256 columns of K, whatever the slab depth: the products of
   // a fused launch and of its halves then add in the same order; a K of an
   // odd number of 64-deep slabs would start the second round of them in the
   // other sum)
-  const int rot = (kRotates || (S::BK <= 256 && a.rotate)) && a.k >= 256 && a.k % 128 == 0
+  const int rot = S::BK <= 256 && a.rotate && a.k >= 256 && a.k % 128 == 0
                       ? tile / kXcds % static_cast<int>(a.k / 256) * (256 / std::min(256, S::BK))
                       : 0;
 
@@ -572,7 +572,10 @@ hipError_t launch_stream(int epi, const StreamPlan &p, const GemmArgs &args, hip
   const int64_t n = epi == kGemmQkvRope  ? a.n0 + a.n1 + a.n2
                     : epi == kGemmSwiglu ? 2 * a.n0
                                          : a.n0;
-  a.rotate = epi == kGemmF32 && p.splits == 1 && n > 65536;
+  if (epi == kGemmSwiglu || epi == kGemmSilu || epi == kGemmMul)
+    a.rotate = 2 * a.n0 > 48 * static_cast<int64_t>(gemm_device_cus(s));
+  else
+    a.rotate = epi == kGemmF32 && p.splits == 1 && n > 65536;
   switch (epi) {
     case kGemmStore:
       return launch_nr<kGemmStore, StreamFms>(p.rows, p.fm, StreamRows{}, a, n, s, 1);
