@@ -27,8 +27,9 @@
 // less over K = 2048, 2.9 more over K = 14336).  Waves 0-3 multiply the even 32-deep chunks of K, waves 4-7 the odd
 // ones, each into two sums in turn, so that no chain of fp32 additions is
 // longer than a quarter of K (error of a product against 64 bits, K = 4096:
-// 1.9e-7 of its norm, with one sum a wave 2.7e-7); a quarter holds the same
-// chunks whatever the shape of the workgroup.  The halves meet in LDS as an
+// 1.9e-7 of its norm, with one sum a wave 2.7e-7, one chain 4.0e-7); a quarter
+// holds the same
+// chunks whatever the shape of the workgroup (of up to 128 tokens).  The halves meet in LDS as an
 // fp32 tile, from which the
 // epilogue takes 4 columns (or 4 RoPE pairs) of a token at a time.
 // Wide SwiGLU launches and the logits of a whole vocabulary start each tile
@@ -94,6 +95,9 @@ struct StreamShape {
   static constexpr int WM = 4 / WN;
   static constexpr int FMW = (FM + WM - 1) / WM;
   static constexpr int FNW = (FN + WN - 1) / WN;
+  // sums of a fragment in a wave (160 tokens: one, half of K; the second cost
+  // 0.6% of a layer of 157 rows)
+  static constexpr int SUMS = FM <= 8 ? 2 : 1;
   static_assert(NR % 8 == 0 && STAGES >= 3 && LDS <= 160 * 1024, "shape");
   static_assert((STAGES - 1) * PER < 64, "vmcnt holds 6 bits");
 };
@@ -202,9 +206,9 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
   const int wm = (wave % 4) / S::WN;
   // waves left without a fragment of their own only load
   const bool idle = S::WM >= 2 * FM && wm >= FM;
-  f32x4 acc[2][S::FMW][S::FNW];  // the half's chunks go to either sum in turn
+  f32x4 acc[S::SUMS][S::FMW][S::FNW];  // the half's chunks go to either sum in turn
 #pragma unroll
-  for (int e = 0; e < 2; ++e)
+  for (int e = 0; e < S::SUMS; ++e)
 #pragma unroll
     for (int i = 0; i < S::FMW; ++i)
 #pragma unroll
@@ -240,7 +244,7 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
     for (int q = 0; q < KS; ++q) {
       if (KS > 1 && 2 * q + kg >= valid) break;
       constexpr int kOdd = decltype(odd)::value;
-      const int set = KS == 1 ? kOdd : q & 1;
+      const int set = S::SUMS == 1 ? 0 : KS == 1 ? kOdd : q & 1;
 #pragma unroll
       for (int i = 0; i < S::FMW; ++i)
 #pragma unroll
@@ -289,10 +293,12 @@ __global__ __launch_bounds__(512) void gemm_stream_kernel(GemmArgs a) {
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
   __syncthreads();
+  if constexpr (S::SUMS == 2) {
 #pragma unroll
-  for (int i = 0; i < S::FMW; ++i)
+    for (int i = 0; i < S::FMW; ++i)
 #pragma unroll
-    for (int j = 0; j < S::FNW; ++j) acc[0][i][j] += acc[1][i][j];
+      for (int j = 0; j < S::FNW; ++j) acc[0][i][j] += acc[1][i][j];
+  }
   float *tile_f = reinterpret_cast<float *>(ring);
   auto each = [&](auto f) {
 #pragma unroll
