@@ -20,9 +20,9 @@
 //                prompts that fill 160-row tiles better than 256-row ones
 //                (129 .. 160, 257 .. 320, 513 .. 640 rows), and split K
 //                where its tiles divide over the CUs more evenly;
-//   GemmTile256  256 x 128, 8 waves, a ring of 3 slab buffers: the large
-//                GEMMs (at least as many 256-row tiles as CUs: q, o, gate,
-//                up, down and the fused gate|up at M = 2048);
+//   GemmTile256  256 x 128, 8 waves, a ring of 3 slab buffers: the other
+//                GEMMs of at least as many 256-row tiles as CUs (q, o, down
+//                and the fused q|k|v at M = 2048);
 //   GemmTile128  128 x 128, 4 waves, a ring of 4;
 //   GemmTile64   64 x 128, 4 waves, a ring of 6: where 128-row tiles would
 //                leave CUs idle (the N = 1024 K / V projections at M = 2048).
@@ -30,9 +30,9 @@
 // When the last round of tiles would leave at least half of the CUs idle,
 // the last tile columns run as tiles of half the height in the same launch
 // (GemmTileWideHalf, 128 x 256, for GemmTileWide; GemmTile128x8 for
-// GemmTile256; GemmTile64 for GemmTile128): M = 2048,
-// N = 14336 runs 768 full tiles in three rounds, then 256 half tiles,
-// instead of three and a half rounds of full tiles.
+// GemmTile256; GemmTile64 for GemmTile128): the fused gate|up (28672 weight
+// rows) at M = 2048 runs 768 of its 896 256 x 256 tiles in three rounds, then
+// 256 half tiles, instead of three and a half rounds of full tiles.
 //
 // Staging.  Slabs move global -> LDS by buffer loads that write LDS
 // themselves (buffer_load_dwordx4 ... lds: no staging registers, no
@@ -901,7 +901,7 @@ __device__ __forceinline__ void gemm_wide_run(const GemmArgs &a, int tm, int tn,
 // round of T tiles would leave at least half of the CUs idle, the last
 // tail_n tile columns with tiles of half the height (TH, the same wave
 // count): those columns then take one round of half tiles instead of a
-// partial round of full ones (M = 2048, N = 14336: 768 full tiles in 3
+// partial round of full ones (M = 2048, fused gate|up: 768 full tiles in 3
 // rounds of 256, then 256 half tiles, instead of 3.5 rounds of full tiles).
 // Workgroup b runs on XCD b % 8 (see "Tile order"); each XCD takes a
 // contiguous range of full tiles first, then of half tiles, so the half

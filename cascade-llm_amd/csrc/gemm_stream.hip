@@ -6,44 +6,42 @@
 // then by what each CU takes in besides, since a CU's loads return in order
 // and the X lines that hit its XCD's L2 queue with the weight lines that do
 // not.  So one workgroup per CU owns a run of weight rows that divides the
-// matrix over the CUs (112 of the 28672 gate and up rows, 24 of the
-// 6144 q|k|v rows, 16 of o_proj's 4096: not a power of two, so these rounds
-// are full; other widths take the next built count, which leaves at most
-// half of the CUs idle: gate|up of 4096, M = 6: 15.1 us on 32 rows, 23.2 on
-// 112; logits of 8192 17.6 on 32, 24.3 on 128) and walks all of K once: the
-// ramp of a launch is paid
-// once, and every token row is read once per workgroup.  Where the token
-// rows would outweigh the weight rows, 2 or 4 workgroups on one XCD take a
-// share of the
-// tokens and twice or four times the weight rows each (stream_plan).
+// matrix over the CUs (112 of the 28672 gate and up rows, 24 of the 6144 q|k|v
+// rows, 16 of o_proj's 4096: not a power of two, so these rounds are full;
+// other widths take the next built count, which leaves at most half of the CUs
+// idle: gate|up of 4096, M = 6: 15.1 us on 32 rows, 23.2 on 112; logits of
+// 8192 17.6 on 32, 24.3 on 128) and walks all of K once: the ramp of a launch
+// is paid once, and every token row is read once per workgroup.  Where the
+// token rows would outweigh the weight rows, 2 or 4 workgroups on one XCD take
+// a share of the tokens and twice or four times the weight rows each
+// (stream_plan).
 //
-// K is walked in slabs through a ring of LDS buffers (buffer loads straight
-// to LDS, up to 148 KB in flight; slab depth 64 to 512 so that a step
-// moves 16 KB or more), nontemporal where one workgroup alone reads the
-// rows.  Up to 16 rows over few columns a launch is a chain of steps with
-// little to load in each: 512-deep slabs halve them, and waves that would
-// repeat another one's fragment leave the LDS alone (M = 6, N = 1024: 8.0 ->
-// 6.8 us, N = 4096 10.0 -> 9.5; without the nontemporal hint 0.5 to 1.0 us
-// less over K = 2048, 2.9 more over K = 14336).  Waves 0-3 multiply the even 32-deep chunks of K, waves 4-7 the odd
-// ones, each into two sums in turn, so that no chain of fp32 additions is
-// longer than a quarter of K (error of a product against 64 bits, K = 4096:
-// 1.9e-7 of its norm, with one sum a wave 2.7e-7, one chain 4.0e-7); a quarter
-// holds the same
-// chunks whatever the shape of the workgroup (of up to 128 tokens).  The halves meet in LDS as an
-// fp32 tile, from which the
+// K is walked in slabs through a ring of LDS buffers (buffer loads straight to
+// LDS, up to 148 KB in flight; slab depth 64 to 512 so that a step moves 16 KB
+// or more), nontemporal where one workgroup alone reads the rows.  Up to 16
+// rows over few columns a launch is a chain of steps with little to load in
+// each: 512-deep slabs halve them, and waves that would repeat another one's
+// fragment leave the LDS alone (M = 6, N = 1024: 8.0 -> 6.8 us, N = 4096 10.0
+// -> 9.5; without the nontemporal hint 0.5 to 1.0 us less over K = 2048, 2.9
+// more over K = 14336).  Waves 0-3 multiply the even 32-deep chunks of K,
+// waves 4-7 the odd ones, each into two sums in turn, so that no chain of fp32
+// additions is longer than a quarter of K (error of a product against 64 bits,
+// K = 4096: 1.9e-7 of its norm, with one sum a wave 2.7e-7, one chain 4.0e-7);
+// a quarter holds the same chunks whatever the shape of the workgroup (of up
+// to 128 tokens).  The halves meet in LDS as an fp32 tile, from which the
 // epilogue takes 4 columns (or 4 RoPE pairs) of a token at a time.
-// Wide SwiGLU launches and the logits of a whole vocabulary start each tile
-// at another run of K: with every CU on the same columns of rows 8 KB apart
-// the same few channels serve all of them (112 rows a CU, loads alone:
-// 44.9 -> 36.2 us); the sums of those launches depend on the start, hence on
-// the tile, within the same bound.  The runs differ between the tiles of one
-// XCD (tile / 8): taken from the tile number itself they agree within an XCD
-// (logits of 26 rows: 259 us, 217 without any, 174 so).  It pays from about
-// 48 weight rows a CU on (gate|up of 7168, M = 33: 27.8 -> 23.1 us; of 4096
-// 16.4 -> 19.1).  The other kinds, and narrower logits, add in one order
-// whatever their width, so that a product does not depend on the columns
-// beside it, though it would shorten them too (14336 columns, M = 6: 24.8 ->
-// 20.6 us).
+//
+// Wide SwiGLU launches and the logits of a whole vocabulary start each tile at
+// another run of K: with every CU on the same columns of rows 8 KB apart the
+// same few channels serve all of them (112 rows a CU, loads alone: 44.9 ->
+// 36.2 us); the sums of those launches depend on the start, hence on the tile,
+// within the same bound.  The runs differ between the tiles of one XCD (tile /
+// 8): taken from the tile number itself they agree within an XCD (logits of 26
+// rows: 259 us, 217 without any, 174 so).  It pays from about 48 weight rows a
+// CU on (gate|up of 7168, M = 33: 27.8 -> 23.1 us; of 4096 16.4 -> 19.1).  The
+// other kinds, and narrower logits, add in one order whatever their width, so
+// that a product does not depend on the columns beside it, though it would
+// shorten them too (14336 columns, M = 6: 24.8 -> 20.6 us).
 //
 // Weights are the A operand, tokens the B operand: a lane then holds 4
 // consecutive weight rows, i.e. output columns, of one token.  8-row blocks
@@ -57,7 +55,7 @@
 // Measured, MI355X, rotating weights, against the kernels it replaced
 // (per launch): M = 6 gate|up 51.2 -> 38.0 us, q|k|v 18.2 -> 12.1; M = 45
 // gate|up 70.1 -> 39.5 (5.9 TB/s), q|k|v 23.1 -> 15.5, o_proj 16.8 -> 13.0,
-// down_proj (4 runs of K) 31.3 -> 27.6 with the reduction; M = 157 gate|up
+// down_proj (4 runs of K) 31.3 -> 26.4 with the reduction; M = 157 gate|up
 // 73.6 -> 59.2, q|k|v 28.7 -> 22.7, o_proj 27.9 -> 17.1, k / v 18 -> 10.7;
 // M = 26 logits of 128256 rows 259 -> 168.
 #include <algorithm>

@@ -49,11 +49,10 @@ def linear_bound_report(actual, x, w):
     (17, 384, 4096), (64, 4096, 4096), (65, 1024, 4096), (128, 4096, 14336),
     (192, 14336, 256), (256, 14336, 192)])
 def test_gemm_matches_oracle(gpu_device, m, n, k):
-    # m <= 16 and m <= 64: the two skinny kernels; m <= 256 over at most 64
-    # column pairs per 64-row block: blocks of the 64-row skinny kernel
-    # (130 x 1024, 128 x 4096, 65 x 1024, 129 x 200); else tiles (128-row
-    # tiles short of a round where 64-row ones would take two: 192 / 256 x
-    # 14336);
+    # up to 160 rows, 256 over at most 6144 columns: the streaming kernel (one
+    # token tile up to 48 rows, two or four past that: 130 x 1024, 128 x 4096,
+    # 65 x 1024, 129 x 200); else tiles (128-row tiles short of a round where
+    # 64-row ones would take two: 192 / 256 x 14336);
     # n = 1001: rows not 16-byte aligned, the element-wise epilogue runs.
     # Slab counts (K / 64): odd and even counts (1, 2, 3, 5, 6, 7, 17, 64,
     # 224) below and above the ring depth of each tile shape (256-row
@@ -78,12 +77,11 @@ def test_gemm_matches_oracle(gpu_device, m, n, k):
 
 @pytest.mark.parametrize("m", [3, 16, 40, 64])
 def test_skinny_single_fragment_equals_column_pairs(gpu_device, m):
-    # At N = 4096 the short-prompt kernels give each 16-column fragment its
-    # own workgroup (the column pairs would fill half the CUs); at
-    # N = 14336 they keep the pairs.  The first 4096 columns of the wide
+    # At N = 4096 the streaming kernel gives a workgroup 16 or 32 columns, at
+    # N = 14336 64 or 112.  The first 4096 columns of the wide
     # product are the narrow product, so the two forms must agree bit for
     # bit, for the plain, residual and fp32 epilogues.
-    print("skinny single-fragment m={}".format(m), flush=True)
+    print("columns of a workgroup m={}".format(m), flush=True)
     dev = gpu_device
     k = 4096
     x = cases.normal_bf16((m, k), 121).to(dev)
@@ -173,7 +171,7 @@ def test_gemm_split_k_matches_oracle(gpu_device, m, n, k):
 
 @pytest.mark.parametrize("m", [5, 37])
 def test_gemm_f32out_matches_float64(gpu_device, m):
-    # m = 5: the skinny kernel's fp32 epilogue; m = 37: 64-row tiles
+    # the streaming kernel's fp32 epilogue, one and three token fragments
     dev = gpu_device
     n, k = 128256 // 8, 4096
     x = cases.normal_bf16((m, k), 103)
@@ -272,15 +270,15 @@ def test_gemm_half_tile_tail_matches_oracle(gpu_device, m, n, k):
 
 
 # Outputs whose schedule of 256 x 256 tiles (two 128-column sub-tiles per
-# workgroup, 32-deep slabs) is shorter than that of 256 x 128 tiles run on
+# workgroup, 64-deep slabs in two buffers) is shorter than that of 256 x 128 tiles run on
 # them: 8000 columns (63 128-column tiles, the last one partial, so the last
 # workgroup's second sub-tile lies past the output; k = 64: fewer slabs
-# than the ring holds), 8192 (one whole round), 600 x 28672 and 2048 x
+# than the buffers hold), 8192 (one whole round), 600 x 28672 and 2048 x
 # 28672 (a last round of 128 x 256 half-height tiles; SwiGLU over 2 x 28672
 # rows: whole rounds, and at m = 600 a partial last round).  The split
 # SwiGLU halves of 8192 / 28672 run on 256 x 128 or 256 x 256 tiles by the
 # same rule, and the fused result equals the split one bit for bit either
-# way (the K order of the MFMAs does not depend on the slab depth).
+# way (every tile adds K in the same order).
 @pytest.mark.parametrize("m,n,k", [(2048, 8000, 64), (2048, 8192, 128),
                                    (600, 28672, 320), (2048, 28672, 64)])
 def test_gemm_wide_tiles_match_oracle(gpu_device, m, n, k):
@@ -437,8 +435,8 @@ def test_qkv_rope_gemm_matches_oracle(gpu_device, m, pos0):
 
 
 # matrix granularity: q, k, v in three launches == one fused launch; at
-# m = 2048 the fused launch takes three heads per tile (32-deep slabs) and
-# the split ones 256 x 128 / 64 x 128 tiles (64-deep), in the same K order
+# m = 2048 the fused launch takes 256 x 128 tiles and a round of half-height
+# ones, the split ones 256 x 128 / 64 x 128 tiles, in the same K order
 @pytest.mark.parametrize("m", [70, 2048])
 def test_qkv_rope_gemm_split_matrices_equal_fused(gpu_device, m):
     dev = gpu_device
