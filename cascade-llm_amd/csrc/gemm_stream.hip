@@ -8,8 +8,7 @@
 // not.  So one workgroup per CU owns a run of weight rows that divides the
 // matrix over the CUs (112 of the 28672 gate and up rows, 24 of the 6144 q|k|v
 // rows, 16 of o_proj's 4096: not a power of two, so these rounds are full;
-// other widths take the next built count, which leaves at most half of the CUs
-// idle: gate|up of 4096, M = 6: 15.1 us on 32 rows, 23.2 on 112; logits of
+// other widths take the next built count, at most twice their share: gate|up of 4096, M = 6: 15.1 us on 32 rows, 23.2 on 112; logits of
 // 8192 17.6 on 32, 24.3 on 128) and walks all of K once: the ramp of a launch
 // is paid once, and every token row is read once per workgroup.  Where the
 // token rows would outweigh the weight rows, 2 or 4 workgroups on one XCD take
@@ -452,12 +451,28 @@ static hipError_t launch_stream_shape(const GemmArgs &args, int64_t n, hipStream
 template <int... V>
 struct Ints {};
 
+// Those a plan can ask for.  Below 64 rows (of both matrices) the token tiles
+// are as many as wanted (stream_plan), so that 4 fragments hold their share;
+// 10 fragments come with more than 64, and for fp32 with partials of split K
+// only (logits stop at 128 tokens).
+constexpr bool stream_built(int epi, int rows, int fm) {
+  if (epi == kGemmQkvRope) return true;
+  const int all = epi == kGemmSilu || epi == kGemmMul ? 2 * rows : rows;
+  if (all < 64) return fm <= 4;
+  return fm < 10 || (all > 64 && (epi != kGemmF32 || rows == 128));
+}
+
 template <int EPI, int NR, int... FMS>
 static hipError_t launch_fm(int fm, Ints<FMS...>, const GemmArgs &a, int64_t n, hipStream_t s,
                             int splits) {
   hipError_t e = static_cast<hipError_t>(CASCADE_ESHAPE);
-  (void)((fm == FMS ? (e = launch_stream_shape<EPI, FMS, NR>(a, n, s, splits), true) : false) ||
-         ...);
+  auto launch = [&](auto shape) {
+    constexpr int kFm = decltype(shape)::value;
+    if constexpr (stream_built(EPI, NR, kFm))
+      e = launch_stream_shape<EPI, kFm, NR>(a, n, s, splits);
+    return true;
+  };
+  (void)((fm == FMS && launch(std::integral_constant<int, FMS>{})) || ...);
   return e;
 }
 
@@ -545,7 +560,7 @@ StreamPlan stream_plan(int epi, int64_t m, int64_t n, int cus) {
   const int64_t fm = (frags + mt - 1) / mt;
   p.fm = epi == kGemmQkvRope ? at_least(StreamFmsQkv{}, fm) : at_least(StreamFms{}, fm);
   p.splits = 1;
-  return p.fm ? p : none;
+  return p.fm && stream_built(epi, p.rows, p.fm) ? p : none;
 }
 
 // down_proj (K = 14336, N = 4096): in one pass each of 256 workgroups would
