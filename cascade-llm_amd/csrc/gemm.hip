@@ -1106,22 +1106,22 @@ static int gemm_check_w(const void *w, int64_t n, int64_t granule, int64_t k) {
 
 using namespace cascade;
 
-// Split K.  Where 256-row tiles would keep at most half of the CUs busy over
-// a long K (K >= 8192; prompts of 17 to 1280 rows over N = 4096: down_proj),
-// K is split over up to kSplitMax rows of workgroups, each writing
-// an fp32 partial tile into the caller's workspace; a second launch sums
-// the partials in split order and applies the element-wise epilogue at the
-// same rounding points as the one-pass tile (bf16(sum), then the residual
-// add).  The partials associate the K sum differently from one pass, so a
-// result may differ from the one-pass tile in the last bf16 place, within
-// the same rounding bound.  Up to 256 rows the streaming kernel writes the
-// partials where it has enough runs (stream_split_plan), past that 256 x 128 tiles, or 160 x 256
-// tiles where, at kLowRound a tile, their more numerous splits are shorter
-// (down_proj: 320 rows 53.7 -> 50.1 us, 613 rows 86.6 -> 73.4, 768 rows
-// 104 -> 92; 1100 and 1280 rows, whose 160 tiles of 256 x 128 do not split,
-// 192 -> 120 and 218 -> 127).  Over a short K (o_proj) one pass ends before
-// a split launch and its reduction (M = 64: 13.8 against 15.2 us;
-// M = 192 .. 1024: 22.0 .. 33.8 against 23.3 .. 42.8).
+// Split K.  Where 256-row tiles would keep at most half of the CUs busy over a
+// long K (K >= 8192; prompts of 17 to 1280 rows over N = 4096: down_proj), K
+// is split over up to kSplitMax rows of workgroups, each writing an fp32
+// partial tile into the caller's workspace; a second launch sums the partials
+// in split order and applies the element-wise epilogue at the same rounding
+// points as the one-pass tile (bf16(sum), then the residual add).  The
+// partials associate the K sum differently from one pass, so a result may
+// differ from the one-pass tile in the last bf16 place, within the same
+// rounding bound.  Up to 256 rows the streaming kernel writes the partials
+// where it has enough runs (stream_split_plan), past that 256 x 128 tiles, or
+// 160 x 256 tiles where, at kLowRound a tile, their more numerous splits are
+// shorter (down_proj: 320 rows 53.7 -> 50.1 us, 613 rows 86.6 -> 73.4, 768
+// rows 104 -> 92; 1100 and 1280 rows, whose 160 tiles of 256 x 128 do not
+// split, 192 -> 120 and 218 -> 127).  Over a short K (o_proj) one pass ends
+// before a split launch and its reduction (M = 64: 13.8 against 15.2 us; M =
+// 192 .. 1024: 22.0 .. 33.8 against 23.3 .. 42.8).
 constexpr int kSplitMax = 8;
 constexpr int kSplitMinSlabs = 8;  // 64-deep slabs per split, at least
 // Of 160 x 256 tiles: their ramp and the reduction of twice the partials

@@ -8,12 +8,12 @@
 // not.  So one workgroup per CU owns a run of weight rows that divides the
 // matrix over the CUs (112 of the 28672 gate and up rows, 24 of the 6144 q|k|v
 // rows, 16 of o_proj's 4096: not a power of two, so these rounds are full;
-// other widths take the next built count, at most twice their share: gate|up of 4096, M = 6: 15.1 us on 32 rows, 23.2 on 112; logits of
-// 8192 17.6 on 32, 24.3 on 128) and walks all of K once: the ramp of a launch
-// is paid once, and every token row is read once per workgroup.  Where the
-// token rows would outweigh the weight rows, 2 or 4 workgroups on one XCD take
-// a share of the tokens and twice or four times the weight rows each
-// (stream_plan).
+// other widths take the next built count, at most twice their share: gate|up
+// of 4096, M = 6: 15.1 us on 32 rows, 23.2 on 112; logits of 8192 17.6 on 32,
+// 24.3 on 128) and walks all of K once: the ramp of a launch is paid once, and
+// every token row is read once per workgroup.  Where the token rows would
+// outweigh the weight rows, 2 or 4 workgroups on one XCD take a share of the
+// tokens and twice or four times the weight rows each (stream_plan).
 //
 // K is walked in slabs through a ring of LDS buffers (buffer loads straight to
 // LDS, up to 148 KB in flight; slab depth 64 to 512 so that a step moves 16 KB
@@ -490,7 +490,7 @@ using StreamFmsQkv = Ints<1, 2, 3, 4, 5>;
 using StreamRows = Ints<16, 32, 64, 112>;              // plain, residual
 using StreamRowsQkv = Ints<16, 24, 32, 48, 64, 96>;
 using StreamRowsSwiglu = Ints<16, 32, 64, 112>;
-using StreamRowsHalf = Ints<8, 16, 32, 56>;                    // silu, mul: half of swiglu's
+using StreamRowsHalf = Ints<8, 16, 32, 56>;            // silu, mul: half of swiglu's
 using StreamRowsF32 = Ints<16, 32, 64, 112, 128>;      // logits; split-K partials
 
 template <int... V>
